@@ -1290,7 +1290,7 @@ static int compact_phase(cbm_ctx* c, int32_t* flag) {
 
 // DGADI sweeps after the reaction step (which wrote R = med_c[1 - cur]); the
 // last sweep lands in C = med_c[cur].  Every sweep writes the interior lines
-// of its destination, then the boundary nodes from the initial field.
+// of its destination and the boundary nodes from the initial field.
 static int adi_sweeps(cbm_ctx* c) {
   double* C = c->med_c[c->med_cur];
   double* R = c->med_c[1 - c->med_cur];
@@ -1312,8 +1312,8 @@ static int adi_sweeps(cbm_ctx* c) {
     a.sub = c->adi_sub; a.main = c->adi_main; a.sup = c->adi_sup;
     a.lines = 1;
     for (int b = 0; b < c->dims; ++b) if (b != ax) a.lines *= n[b] - 2;
+    a.init = c->med_init;
     HIPCHK(c, launch_adi_sweep(c->stream, a));
-    HIPCHK(c, launch_adi_border(c->stream, dst[ax], c->med_init, n, c->dims, c->med_nodes));
   }
   return CBM_OK;
 }

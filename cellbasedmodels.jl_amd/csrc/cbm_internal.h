@@ -121,7 +121,14 @@ struct AdiArgs {
   int32_t dims, axis;
   double sub, main, sup;
   int64_t lines;
+  const double* init;   // the initial field, held on every boundary node of dst
+  int64_t nblk;         // blocks on lines; the launch's further blocks write boundary faces
+  int32_t lpb, lds_ld;  // lines per block and their LDS stride (k_adi_lines)
 };
+
+// LDS of a k_adi_lines block (lines and tables): two blocks per CU
+constexpr int64_t ADI_LDS_BYTES = 64 * 1024;
+constexpr int ADI_U = 8;    // nodes of a line in registers at a time
 
 struct ExportArgs {
   StageArgs s;
@@ -178,10 +185,8 @@ hipError_t launch_disp_check(int dims, int nblocks, int block, hipStream_t s, co
 hipError_t launch_medium_inject(hipStream_t s, double* c, unsigned long long* add, int64_t nodes);
 hipError_t launch_medium_count(int nblocks, int block, hipStream_t s, const MediumArgs& a);
 hipError_t launch_medium_step(hipStream_t s, const MediumArgs& a);
+// one sweep, and the boundary nodes of dst (any coordinate 0 or n-1) from init
 hipError_t launch_adi_sweep(hipStream_t s, const AdiArgs& a);
-// boundary nodes of dst (any coordinate 0 or n-1) set from init
-hipError_t launch_adi_border(hipStream_t s, double* dst, const double* init, const int32_t* n, int32_t dims,
-                             int64_t nodes);
 
 hipError_t launch_rule_decide(int nblocks, int block, hipStream_t s, const RuleArgs& a);
 // copies positions, vol and the user parameters of the committed agents into
