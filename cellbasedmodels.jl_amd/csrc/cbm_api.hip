@@ -155,7 +155,12 @@ struct cbm_ctx {
   int bdim[3] = {1, 1, 1};
   int brick_cap = 0;                      // agents staged per brick block
   size_t brick_lds = 0;                   // its LDS bytes
+  size_t brick_lds_user = 0;              // and those of a hipRTC module's brick kernel (one lane per agent)
+  int brick_g = 1;                        // lanes per agent in the cell-linked stage
   int32_t* bricks2 = nullptr;             // sub-bricks for dense regions (StageArgs::brick2)
+  int32_t* sub_first = nullptr;           // main brick -> its sub-bricks (BrickSrc::sub_first, sub_ids)
+  int32_t* sub_ids = nullptr;
+  int32_t* sub_list = nullptr;            // the launch's work list and, after it, its length
   int64_t nbricks2 = 0;
   int bdim2[3] = {1, 1, 1};
   int brick_cap2 = 0;
@@ -418,28 +423,60 @@ static void brick_table(cbm_ctx* c, const int* bd, std::vector<int32_t>& tab) {
 // its rows are one range).  m is the largest size whose expected population
 // (the densest simulation's mean density; capacity when rules change the
 // population) stays within ~1.25 blocks of 256 threads, lowered while the
-// LDS for 1.2x the expected halo population would exceed 64 KiB (a denser
-// brick is left to the row-parallel stage kernel).  Bricks
-// are listed per simulation in Morton order of their coordinates.
+// LDS for 1.2x the expected halo population would exceed 44 KiB, so that
+// three or four blocks share a CU (a denser brick is left to the
+// row-parallel stage kernel).  The density is that of
+// the box: an open grid's outer cells hold no agents, and counting them put
+// the tiles of small boxes under what their interior holds (120,001 soft
+// spheres, 32^3 cells: every interior brick overflowed, 123 us per stage in
+// the row kernel beside 75 us on bricks).  Bricks are listed per simulation
+// in Morton order of their coordinates.
+//
+// Where rules add agents the main bricks are half that size: what does not
+// fit goes to sub-bricks, and a sparse edge of the colony is done sooner
+// (150,001 agents at 2 per unit area: 23 us for the main bricks against 32).
+// Elsewhere, past one block's population, m is lowered while there are fewer
+// than 256 bricks and more than 64 agents per brick.
+//
+// A brick walks its agents with one lane each when it holds about a block of
+// them, else with four (brick_one): 13-20 % more instructions, but no idle
+// lanes and shorter walks.  One against four lanes per agent, us per stage:
+// 238 agents a brick in 3,312 3-D bricks 135 / 165, 195 in 1,540 2-D bricks
+// 38 / 53, 190 in 289 2-D bricks 22 / 27; 51 in 392 2-D bricks 40 / 18, 54 in
+// 36 19 / 16, 157 soft spheres in 1,024 3-D bricks 114 / 81.  In space the
+// walk of 27 cells is the longer part, and while the bricks do not fill the
+// chip its latency counts: 232 agents in 432 bricks 59 / 46.
+constexpr double BRICK_ONE_LANE = 160.0;      // agents per brick from which a lane walks an agent
+constexpr double BRICK_ONE_LANE_3D = 1024.0;  // and, in space, the number of bricks
+
 static int setup_bricks(cbm_ctx* c) {
   const int D = c->dims;
   const bool soft = c->inertial;
-  double rho = 0.0;
+  double rho = 0.0, agents = 0.0, cells = 0.0;
   for (int s = 0; s < c->S; ++s) {
     const double n = (double)std::max<int64_t>(c->rules ? c->sims[s].n_max : c->sims[s].n, 1);
-    rho = std::max(rho, n / (double)c->h_sims[s].ncells);
+    const SimDev& sd = c->h_sims[s];
+    double inner = 1.0;                 // cells of the box itself
+    for (int a = 0; a < D; ++a) inner *= std::max(1.0, std::min((double)sd.gn[a], sd.L[a] / sd.gedge[a]));
+    rho = std::max(rho, n / inner);
+    agents += n;
+    cells += (double)sd.ncells;
   }
   const int mmin = D, mmax = D == 3 ? 9 : 10;
   int m = mmin;
-  while (m < mmax && rho * (double)(1 << (m + 1)) <= 320.0) ++m;
-  const int64_t budget = 64 * 1024;
+  while (m < mmax && rho * (double)(1 << (m + 1)) <= (c->rules ? 160.0 : 320.0)) ++m;
+  if (!c->rules && agents > 256.0) {
+    const double want = std::min(256.0, agents / 64.0);
+    while (m > mmin && cells / (double)(1 << m) < want) --m;
+  }
+  const int64_t budget = 44 * 1024, budget2 = 64 * 1024;   // main bricks, sub-bricks
   // LDS bytes per staged agent and in all of a tile: the Verlet list build
   // stages positions and slots, the cell-linked stage positions (and radius
   // and fate for soft spheres); both add an owner and a home-row index
   const bool build = c->verlet || c->clv;   // the bricks serve the list build
   const int64_t per = build ? 8 * D + 4 + 4 : 8 * (D + (soft ? 1 : 0)) + (soft ? 4 : 0) + 4;
-  auto tile_bytes = [&](int cp, int H) {
-    return build ? vbrick_lds_bytes(D, cp, H) : brick_lds_bytes(D, soft, cp, H);
+  auto tile_bytes = [&](int cp, int H, int g = 4, bool sub = false) {
+    return build ? vbrick_lds_bytes(D, cp, H) : brick_lds_bytes(D, soft, cp, H, g, sub);
   };
   int bd[3] = {1, 1, 1};
   int cap = 0;
@@ -461,7 +498,10 @@ static int setup_bricks(cbm_ctx* c) {
   }
   for (int a = 0; a < 3; ++a) c->bdim[a] = bd[a];
   c->brick_cap = cap;
-  c->brick_lds = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]));
+  const double per_brick = rho * (double)(1 << m), bricks = cells / (double)(1 << m);
+  c->brick_g = c->rules || per_brick < BRICK_ONE_LANE || (D == 3 && bricks < BRICK_ONE_LANE_3D) ? 4 : 1;
+  c->brick_lds = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]), c->brick_g);
+  c->brick_lds_user = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]), 1);
   std::vector<int32_t> tab;
   brick_table(c, bd, tab);
   c->nbricks = (int64_t)tab.size() / BRICK_WORDS;
@@ -479,18 +519,34 @@ static int setup_bricks(cbm_ctx* c) {
       int b2[3];
       edges(m2, b2);
       const int H2 = brick_halo_cells(D, b2[0], b2[1], b2[2]);
-      const int64_t capmax = (budget - tile_bytes(0, H2) - 16) / per;
+      const int64_t capmax = (budget2 - tile_bytes(0, H2, 1, true) - 16) / per;
       const double want = 1.2 * SUB_BRICK_DENSITY * H2 + 32.0;
       if (want > (double)capmax) continue;
       for (int a = 0; a < 3; ++a) c->bdim2[a] = b2[a];
       c->brick_cap2 = (int)std::min<int64_t>(capmax, (int64_t)std::max(256.0, want));
-      c->brick_lds2 = (size_t)tile_bytes(c->brick_cap2, H2);
+      c->brick_lds2 = (size_t)tile_bytes(c->brick_cap2, H2, 1, true);
       std::vector<int32_t> tab2;
       brick_table(c, b2, tab2);
       c->nbricks2 = (int64_t)tab2.size() / BRICK_WORDS;
       if (c->nbricks2 > ((int64_t)1 << 31) - 1) return fail(c, CBM_ERR_CONFIG, "too many cell bricks; raise cellEdge");
       HIPCHK(c, dalloc(&c->bricks2, (int64_t)tab2.size()));
       HIPCHK(c, hipMemcpy(c->bricks2, tab2.data(), sizeof(int32_t) * tab2.size(), hipMemcpyHostToDevice));
+      // the sub-bricks of every main brick (rules: one simulation)
+      int64_t nb[3];
+      for (int a = 0; a < 3; ++a) nb[a] = (c->h_sims[0].gn[a] + bd[a] - 1) / bd[a];
+      std::vector<int32_t> at((size_t)c->nbricks), first((size_t)c->nbricks + 1, 0), ids((size_t)c->nbricks2);
+      auto cell_brick = [&](const int32_t* o) { return o[0] / bd[0] + nb[0] * (o[1] / bd[1] + nb[1] * (o[2] / bd[2])); };
+      for (int64_t b = 0; b < c->nbricks; ++b) at[(size_t)cell_brick(&tab[(size_t)(b * BRICK_WORDS + 1)])] = (int32_t)b;
+      auto main_of = [&](int64_t q) { return at[(size_t)cell_brick(&tab2[(size_t)(q * BRICK_WORDS + 1)])]; };
+      for (int64_t q = 0; q < c->nbricks2; ++q) first[(size_t)main_of(q) + 1]++;
+      for (int64_t b = 0; b < c->nbricks; ++b) first[(size_t)b + 1] += first[(size_t)b];
+      std::vector<int32_t> put(first.begin(), first.end() - 1);
+      for (int64_t q = 0; q < c->nbricks2; ++q) ids[(size_t)put[(size_t)main_of(q)]++] = (int32_t)q;
+      HIPCHK(c, dalloc(&c->sub_first, (int64_t)first.size()));
+      HIPCHK(c, hipMemcpy(c->sub_first, first.data(), sizeof(int32_t) * first.size(), hipMemcpyHostToDevice));
+      HIPCHK(c, dalloc(&c->sub_ids, (int64_t)ids.size()));
+      HIPCHK(c, hipMemcpy(c->sub_ids, ids.data(), sizeof(int32_t) * ids.size(), hipMemcpyHostToDevice));
+      HIPCHK(c, dalloc(&c->sub_list, c->nbricks2 + 1));
       break;
     }
   }
@@ -661,7 +717,8 @@ static void destroy_ctx(cbm_ctx* c) {
   F(c->med_init); F(c->med_tmp); F(c->adi_tab[0]); F(c->adi_tab[1]); F(c->adi_tab[2]);
   F(c->key); F(c->lin); F(c->gbucket); F(c->cell_range); F(c->count); F(c->cursor); F(c->start); F(c->tmp); F(c->cell_row);
   F(c->emax); F(c->wlist); F(c->wlist_n); F(c->fix_rows); F(c->fix_n);
-  F(c->scan_status); F(c->scan_ticket); F(c->list); F(c->list_n); F(c->bricks); F(c->bricks2); F(c->brick_skip); F(c->blk_flag); F(c->flags); F(c->counters);
+  F(c->scan_status); F(c->scan_ticket); F(c->list); F(c->list_n); F(c->bricks); F(c->bricks2);
+  F(c->sub_first); F(c->sub_ids); F(c->sub_list); F(c->brick_skip); F(c->blk_flag); F(c->flags); F(c->counters);
   for (cbm_ctx::DevBuf* b : {&c->adj_tgt, &c->adj_tbase, &c->adj_invn, &c->adj_ck, &c->adj_seg, &c->adj_lam,
                              &c->adj_gpart, &c->adj_lpart}) F(b->p);
   for (int32_t* p : c->snap_l) F(p);
@@ -1064,6 +1121,9 @@ static StageArgs stage_base(cbm_ctx* c) {
   a.brick_over = (unsigned long long*)(c->counters + 2);
   for (int q = 0; q < 3; ++q) a.bdim[q] = c->bdim[q];
   a.brick_cap = c->brick_cap;
+  a.brick_g = c->brick_g;
+  a.sub_first = c->sub_first; a.sub_ids = c->sub_ids;
+  a.sub_list = c->sub_list; a.sub_n = c->sub_list ? c->sub_list + c->nbricks2 : nullptr;
   a.brick2 = c->bricks2; a.nbricks2 = c->nbricks2; a.brick_lds2 = (int64_t)c->brick_lds2;
   for (int q = 0; q < 3; ++q) a.bdim2[q] = c->bdim2[q];
   a.brick_cap2 = c->brick_cap2;
@@ -1149,11 +1209,12 @@ static hipError_t stage_launch(cbm_ctx* c, const StageArgs& a) {
   hipFunction_t f = c->user_fn[noise];
   if (!f) return hipErrorInvalidDeviceFunction;
   StageArgs copy = a;
+  copy.sub_list = nullptr;   // the module has no sub-brick launch
   void* params[] = {(void*)&copy};
   if (c->user_nb == NB_CELL) {
     if (!c->user_brick[noise]) return hipErrorInvalidDeviceFunction;
     const hipError_t e = hipModuleLaunchKernel(c->user_brick[noise], (unsigned)c->nbricks, 1, 1, (unsigned)c->block,
-                                               1, 1, (unsigned)c->brick_lds, c->stream, params, nullptr);
+                                               1, 1, (unsigned)c->brick_lds_user, c->stream, params, nullptr);
     if (e != hipSuccess) return e;
   }
   return hipModuleLaunchKernel(f, (unsigned)c->nblocks, 1, 1, (unsigned)c->block, 1, 1, 0, c->stream, params, nullptr);

@@ -60,10 +60,17 @@ __global__ __launch_bounds__(256) void k_rods(StageArgs a) {
 }
 
 // cell-linked stage on LDS brick tiles (dynamic LDS: brick_lds_bytes)
-template <int D, int LAW, int PER, int NOISE>
-__global__ __launch_bounds__(256) void k_brick(StageArgs a) {
+// G lanes per agent; at most 128 registers, so that four blocks share a CU
+template <int D, int LAW, int PER, int NOISE, int G>
+__global__ __launch_bounds__(256, 4) void k_brick(StageArgs a) {
   extern __shared__ unsigned char brick_lds[];
-  brick_body<D, PairLaw<LAW>, PER, NOISE>(a, brick_lds);
+  brick_body<D, PairLaw<LAW>, PER, NOISE, G>(a, brick_lds);
+}
+
+template <int D, int LAW, int PER, int NOISE>
+__global__ __launch_bounds__(256, 4) void k_sub_brick(StageArgs a) {
+  extern __shared__ unsigned char brick_lds[];
+  sub_brick_body<D, PairLaw<LAW>, PER, NOISE>(a, brick_lds);
 }
 
 // list stage with the pair work flattened over the block (dynamic LDS:
@@ -1318,33 +1325,39 @@ __global__ __launch_bounds__(256) void k_clcell(StageArgs a) {
 // ------------------------------------------------------------- launchers
 struct StageLaunch { dim3 grid, bgrid, block; size_t lds; hipStream_t s; };   // bgrid: one block per brick
 
+template <int D, int PER, int NOISE, int G>
+static hipError_t launch_brick(int law, dim3 grid, dim3 block, size_t lds, hipStream_t s, const StageArgs& a) {
+  switch (law) {
+    case LAW_LINEAR: hipLaunchKernelGGL((k_brick<D, LAW_LINEAR, PER, NOISE, G>), grid, block, lds, s, a); break;
+    case LAW_REP_ADH: hipLaunchKernelGGL((k_brick<D, LAW_REP_ADH, PER, NOISE, G>), grid, block, lds, s, a); break;
+    case LAW_AGGREGATION: hipLaunchKernelGGL((k_brick<D, LAW_AGGREGATION, PER, NOISE, G>), grid, block, lds, s, a); break;
+    case LAW_SOFT_SPHERES: hipLaunchKernelGGL((k_brick<D, LAW_SOFT_SPHERES, PER, NOISE, G>), grid, block, lds, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <int D, int NB, int PER, int NOISE>
 static hipError_t launch_stage_law(int law, const StageLaunch& L, const StageArgs& a) {
   if (NB == NB_CELL) {
     // bricks that fit in LDS, then the rows of those that did not
-    switch (law) {
-      case LAW_LINEAR: hipLaunchKernelGGL((k_brick<D, LAW_LINEAR, PER, NOISE>), L.bgrid, L.block, L.lds, L.s, a); break;
-      case LAW_REP_ADH: hipLaunchKernelGGL((k_brick<D, LAW_REP_ADH, PER, NOISE>), L.bgrid, L.block, L.lds, L.s, a); break;
-      case LAW_AGGREGATION: hipLaunchKernelGGL((k_brick<D, LAW_AGGREGATION, PER, NOISE>), L.bgrid, L.block, L.lds, L.s, a); break;
-      case LAW_SOFT_SPHERES: hipLaunchKernelGGL((k_brick<D, LAW_SOFT_SPHERES, PER, NOISE>), L.bgrid, L.block, L.lds, L.s, a); break;
-      default: return hipErrorInvalidValue;
-    }
-    hipError_t e = hipGetLastError();
+    hipError_t e = a.brick_g == 1 ? launch_brick<D, PER, NOISE, 1>(law, L.bgrid, L.block, L.lds, L.s, a)
+                                  : launch_brick<D, PER, NOISE, 4>(law, L.bgrid, L.block, L.lds, L.s, a);
     if (e != hipSuccess) return e;
     if (a.brick2 && a.nbricks2 > 0) {
-      // the sub-bricks of the bricks that did not fit
+      // the sub-bricks of the bricks that did not fit, from the list
+      // (brick_body): enough blocks to fill the chip at the tile's LDS
       StageArgs b = a;
       b.brick = a.brick2;
       for (int q = 0; q < 3; ++q) b.bdim[q] = a.bdim2[q];
       b.brick_cap = a.brick_cap2;
-      b.brick_sub = 1;
-      const dim3 g2((unsigned)a.nbricks2);
+      const dim3 g2((unsigned)(a.nbricks2 < 1024 ? a.nbricks2 : 1024));
       const size_t lds2 = (size_t)a.brick_lds2;
-      switch (law) {
-        case LAW_LINEAR: hipLaunchKernelGGL((k_brick<D, LAW_LINEAR, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
-        case LAW_REP_ADH: hipLaunchKernelGGL((k_brick<D, LAW_REP_ADH, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
-        case LAW_AGGREGATION: hipLaunchKernelGGL((k_brick<D, LAW_AGGREGATION, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
-        default: hipLaunchKernelGGL((k_brick<D, LAW_SOFT_SPHERES, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
+      switch (law) {   // (soft spheres take no rules)
+        case LAW_LINEAR: hipLaunchKernelGGL((k_sub_brick<D, LAW_LINEAR, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
+        case LAW_REP_ADH: hipLaunchKernelGGL((k_sub_brick<D, LAW_REP_ADH, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
+        case LAW_AGGREGATION: hipLaunchKernelGGL((k_sub_brick<D, LAW_AGGREGATION, PER, NOISE>), g2, L.block, lds2, L.s, b); break;
+        default: return hipErrorInvalidValue;
       }
       e = hipGetLastError();
       if (e != hipSuccess) return e;

@@ -595,6 +595,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a) {
   if (a.gate && *a.gate != a.gate_run) return;
   if (NB == NB_CELL) {
     // cell-linked: only blocks holding rows of bricks too dense for LDS
+    if (a.sub_list && blockIdx.x == 0 && threadIdx.x == 0) *a.sub_n = 0;   // the sub-brick launch is done
     const int b = xcd_tile((int)blockIdx.x, (int)gridDim.x);
     if (!a.blk_flag[b]) return;
     __syncthreads();
@@ -716,9 +717,10 @@ __device__ __forceinline__ void user_stage(const StageArgs& a) {
 // The pair term of one list entry: what pair_into adds to the accumulator,
 // returned instead (+0 for an inactive pair; the accumulator never holds
 // -0, so adding +0 or -0 leaves it unchanged and the sums equal pair_into's).
-template <int D, class Law, int PER>
+template <int D, class Law, int PER, bool SOFT = false>
 __device__ __forceinline__ void pair_term(const Law& law, const double* xi, const double* xj, const double* L,
-                                          const double* hL, double* t) {
+                                          const double* hL, double* t, double rad_i = 0.0, double rad_j = 0.0,
+                                          int64_t fate_i = 0, int64_t fate_j = 0) {
   double dx[3];
 #pragma unroll
   for (int c = 0; c < D; ++c) {
@@ -730,8 +732,14 @@ __device__ __forceinline__ void pair_term(const Law& law, const double* xi, cons
   if (D > 2) s2 = s2 + dx[2] * dx[2];
   const double d = sqrt(s2);
   double s;
-  const bool on = law(d, s);
-  if (Law::per_axis_division) {
+  bool on;
+  if constexpr (SOFT) on = law.pair(d, rad_i, rad_j, fate_i, fate_j, s);
+  else on = law(d, s);
+  if constexpr (SOFT) {
+    // ((s dx) / d) per axis, the reference's order (softSpheres.jl:28-29)
+#pragma unroll
+    for (int c = 0; c < D; ++c) t[c] = on ? (s * dx[c]) / d : 0.0;
+  } else if (Law::per_axis_division) {
 #pragma unroll
     for (int c = 0; c < D; ++c) t[c] = on ? s * (dx[c] / d) : 0.0;
   } else {
@@ -845,9 +853,6 @@ __device__ __forceinline__ int brick_stage(const BrickSrc& src, int b, BrickTile
   t.r0 = src.bucket_start[bt[4]];
   t.r1 = src.bucket_start[bt[5]];
   if (t.r0 >= t.r1) return 0;
-  // a sub-brick whose main brick was staged: nothing left here (a main
-  // brick marks all its rows or none, and this brick lies inside one)
-  if (src.sub && !src.brick_skip[t.r0]) return 0;
   t.B[0] = src.bdim[0]; t.B[1] = D > 1 ? src.bdim[1] : 1; t.B[2] = D > 2 ? src.bdim[2] : 1;
   t.HX = t.B[0] + 2;
   t.HY = D > 1 ? t.B[1] + 2 : 1;
@@ -938,6 +943,20 @@ __device__ __forceinline__ int brick_stage(const BrickSrc& src, int b, BrickTile
     const int64_t q0 = src.block_off[t.sim] + ((int64_t)r0 - sd.row_off) / nt;
     const int64_t q1 = src.block_off[t.sim] + ((int64_t)r1 - 1 - sd.row_off) / nt;
     for (int64_t q = q0 + tid; q <= q1; q += nt) src.blk_flag[q] = 1;
+    if (src.sub_list) {   // or, before it, the sub-brick launch
+      const int32_t e = src.sub_first[b + 1];
+      for (int32_t k0 = src.sub_first[b]; k0 < e; k0 += nt) {
+        const int32_t k = k0 + tid;
+        const int32_t id = k < e ? src.sub_ids[k] : 0;
+        const int32_t* sb = src.sub_brick + BRICK_WORDS * (int64_t)id;
+        const bool rows = k < e && src.bucket_start[sb[4]] < src.bucket_start[sb[5]];
+        const unsigned long long m = __ballot(rows);     // one atomic per wavefront
+        int32_t at = 0;
+        if (rows && (m & ((1ull << (tid & 63)) - 1ull)) == 0ull) at = atomicAdd(src.sub_n, (int32_t)__popcll(m));
+        at = __shfl(at, m ? __ffsll(m) - 1 : 0, 64);
+        if (rows) src.sub_list[at + __popcll(m & ((1ull << (tid & 63)) - 1ull))] = id;
+      }
+    }
     return 2;
   }
 
@@ -1036,18 +1055,68 @@ __device__ __forceinline__ void brick_walk(const BrickTile& t, int h, Visit&& vi
   }
 }
 
-template <int D, class Law, int PER, int NOISE, class Noise = ConstNoise>
-__device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* lds) {
+// The value of lane G of this lane's quad (four consecutive lanes, all active).
+template <int G>
+__device__ __forceinline__ double quad_lane(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), G * 0x55, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), G * 0x55, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// The candidates of a home agent in halo cell h in walk order, G at a time:
+// lane sub of the agent's G lanes gets candidate k + sub of each round (not
+// live past the last one).
+template <int D, int G>
+struct BrickWalk {
+  int32_t ncand, k, q, qe;
+  int ry, hb;
+  __device__ __forceinline__ BrickWalk(const BrickTile& t, int h, int sub)
+      : ncand(brick_ncand<D>(t, h)), k(0), ry(0), hb(brick_run0<D>(t, h)) {
+    q = t.hs[hb] + sub;
+    qe = t.hs[hb + 3];
+  }
+  __device__ __forceinline__ bool more() const { return k < ncand; }
+  __device__ __forceinline__ int32_t next(const BrickTile& t, int sub, bool& live) {
+    live = G == 1 || k + sub < ncand;
+    if (live)
+      while (q >= qe) {   // into the run that holds this candidate; there is one
+        const int32_t past = q - qe;
+        if (++ry == 3) { ry = 0; hb += t.HX * t.HY - 2 * t.HX; } else { hb += t.HX; }
+        q = t.hs[hb] + past;
+        qe = t.hs[hb + 3];
+      }
+    const int32_t at = live ? q : 0;
+    q += G;
+    k += G;
+    return at;
+  }
+};
+
+// The cell-linked stage of a brick.  Built-in laws filter the candidates: a
+// cheap test queues the LDS indices of the pairs within the law's reach (in
+// walk order), and the full pair body runs on those only.  Every pair left
+// out is inactive, so the sum is unchanged.  A full queue is drained and
+// refilled, so cells of any density are tested once; a queue that could only
+// overflow made its lane walk all candidates again with the full body, which
+// soft spheres (15 of 132 candidates near enough, 12 queue entries) did in
+// every wavefront: 172 us per stage for 120,001 of them, 81 us now.
+//
+// G lanes share an agent: they test G consecutive candidates at once and
+// evaluate G queued pairs at once, whose terms the first lane adds in order
+// (DPP moves), so the sums keep the reference's order.  With four, a
+// wavefront waits for the longest walk of 16 agents and not of 64, bricks of
+// fewer agents than lanes keep the lanes busy, and neighboring lanes read
+// neighboring LDS words; the moves and shared adds cost instructions, so
+// bricks that fill their lanes by themselves use one (setup_bricks).
+template <int D, class Law, int PER, int NOISE, int G, bool SUB, class Noise>
+__device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds, int b) {
   constexpr bool SOFT = same_type<Law, PairLaw<LAW_SOFT_SPHERES>>::value;
-  // Built-in laws walk the candidates twice: a cheap pass keeps the LDS
-  // indices of the pairs within the law's reach (in walk order, up to
-  // BRICK_LIST per lane in an LDS queue), and the full pair body runs on
-  // those only.  Every pair left out is inactive, so the sum is unchanged.
-  constexpr bool FILTER = SOFT || has_reach<Law>::value;
+  // on sub-bricks in the plane every candidate takes the pair body: a third
+  // of them is in reach, and the filter costs as much as it saves
+  constexpr bool FILTER = (SOFT || has_reach<Law>::value) && !(SUB && D < 3);
   constexpr int U4 = 4;               // loads issued together per thread while staging
   // stage-2 lists (built-in laws without per-agent radii)
   constexpr bool WL = FILTER && !SOFT;
-  if (a.gate && *a.gate != a.gate_run) return;
   const bool wl = WL && a.wlist != nullptr;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int cap = a.brick_cap;
@@ -1056,7 +1125,9 @@ __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* ld
   src.cell_range = a.cell_range; src.cap = cap;
   for (int e = 0; e < 3; ++e) src.bdim[e] = a.bdim[e];
   src.brick_skip = a.brick_skip; src.blk_flag = a.blk_flag; src.brick_over = a.brick_over;
-  src.sub = a.brick_sub;
+  src.sub = SUB ? 1 : 0;
+  src.sub_first = a.sub_first; src.sub_ids = a.sub_ids; src.sub_brick = a.brick2;
+  src.sub_list = SUB ? nullptr : a.sub_list; src.sub_n = a.sub_n;
   const int H = brick_halo_cells(D, a.bdim[0], D > 1 ? a.bdim[1] : 1, D > 2 ? a.bdim[2] : 1);
 
   BrickTile t;
@@ -1073,8 +1144,8 @@ __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* ld
   p += (size_t)4 * (H + 1);
   t.hrow = (int32_t*)p;
   p += (size_t)4 * H;
-  uint16_t* lst = (uint16_t*)p;       // per-lane queue of kept candidates, entry u at [u * nt + tid]
-  p += (size_t)2 * BRICK_LIST * BRICK_MAX_BLOCK;
+  uint16_t* lst = (uint16_t*)p;       // the agents' queues of kept candidates
+  if (FILTER) p += (size_t)2 * brick_queue(G) * (BRICK_MAX_BLOCK / G);
   t.owner = (uint16_t*)p;
   p += (size_t)2 * cap;
   t.home_li = (uint16_t*)p;
@@ -1088,7 +1159,6 @@ __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* ld
   cols.xi = a.fate;
   cols.xi_lds = fate;
   double rmax = 0.0;
-  const int b = xcd_tile((int)blockIdx.x, (int)gridDim.x);
   const int staged = brick_stage<D, PER, U4, SOFT, SOFT ? BX_I64 : BX_NONE>(src, b, t, cols, rmax);
   if (staged == 2 && wl && tid == 0) *a.lgate = 0;   // its rows get no list
   if (staged != 1) return;
@@ -1100,7 +1170,7 @@ __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* ld
   const uint16_t* owner = t.owner;
   const uint16_t* home_li = t.home_li;
 
-  // 4. the home agents, one per thread
+  // 4. the home agents
   const int32_t nh = t.r1 - t.r0;
   const Law law(sd.p);
   double L[3], hL[3];
@@ -1117,87 +1187,168 @@ __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* ld
       disp2 = half > 0.0 ? half * half : 0.0;
     }
   }
-  for (int32_t k = tid; k < nh; k += nt) {
-    const int32_t li = home_li[k];
-    const int h = owner[li] & 0x7FFF;
-    const int64_t i = (int64_t)hrow[h] + (li - hs[h]);
-    if (a.brick_sub) a.brick_skip[i] = 0;   // done here, not by the row kernel
-    if (i - sd.row_off >= N) continue;
-    double xi[3] = {0.0, 0.0, 0.0};
-    double acc[3] = {0.0, 0.0, 0.0};
-    double upre[3] = {0.0, 0.0, 0.0};
+  auto row_of = [&](int32_t q) {
+    const int hq = owner[q] & 0x7FFF;
+    return (int64_t)hrow[hq] + (q - hs[hq]);
+  };
+  // Each wavefront takes consecutive home agents, 64 at most: it walks them
+  // 16 at a time, four lanes per agent, and then finishes the stage of all of
+  // them with one agent per lane.  `own` is this lane's agent of the finish.
+  const int lane = tid & 63, sub = lane & (G - 1), wv = tid >> 6, nw = nt >> 6;
+  for (int32_t k0 = 0; k0 < nh; k0 += nt) {
+    const int32_t m = nh - k0 < nt ? nh - k0 : nt;
+    const int32_t npw = (m + nw - 1) / nw;            // agents per wavefront
+    const int32_t w0 = k0 + wv * npw;
+    const int32_t w1 = w0 + npw < k0 + m ? w0 + npw : k0 + m;
+    const int32_t own = w0 + lane;
+    int64_t i = -1;
+    int32_t own_li = 0;
+    double upre[3] = {0.0, 0.0, 0.0}, acc[3] = {0.0, 0.0, 0.0};
+    if (own < w1) {
+      own_li = home_li[own];
+      i = row_of(own_li);
+      if (SUB) a.brick_skip[i] = 0;   // done here, not by the row kernel
+      if (i - sd.row_off >= N) i = -1;
+    }
+    if (i >= 0) {
 #pragma unroll
-    for (int c = 0; c < D; ++c) upre[c] = a.U[c][i];   // consumed after the walk
-    {
+      for (int c = 0; c < D; ++c) upre[c] = a.U[c][i];   // consumed after the walk
+    }
+    for (int32_t g0 = w0; g0 < w1; g0 += 64 / G) {
+      const int32_t k = g0 + lane / G;
+      double sum[3] = {0.0, 0.0, 0.0};
+      if (k < w1) {
+        const int32_t li = home_li[k];
+        const int h = owner[li] & 0x7FFF;
+        const int64_t row = row_of(li);
+        double xi[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-      for (int c = 0; c < D; ++c) xi[c] = pos[c][li];
-      const double rad_i = SOFT ? rad[li] : 0.0;
-      const int64_t fate_i = SOFT ? fate[li] : 0;
-      double keep2 = reach2;
-      if constexpr (SOFT) keep2 = law.mu >= 0.0 ? reach2_bound(law.mu * (rad_i + rmax)) : __builtin_inf();
-      auto walk = [&](auto&& visit) { brick_walk<D>(t, h, visit); };
-      auto body = [&](int32_t q, bool live) {
-        double xj[3] = {0.0, 0.0, 0.0};
+        for (int c = 0; c < D; ++c) xi[c] = pos[c][li];
+        const double rad_i = SOFT ? rad[li] : 0.0;
+        const int64_t fate_i = SOFT ? fate[li] : 0;
+        double keep2 = reach2;
+        if constexpr (SOFT) keep2 = law.mu >= 0.0 ? reach2_bound(law.mu * (rad_i + rmax)) : __builtin_inf();
+        BrickWalk<D, G> w(t, h, sub);
+        // G candidates' terms (this lane's is q's, nothing unless live) added
+        // to the agent's sum, in their order, by its first lane
+        auto add = [&](int32_t q, bool live) {
+          double xj[3] = {0.0, 0.0, 0.0}, t[3];
 #pragma unroll
-        for (int c = 0; c < D; ++c) xj[c] = pos[c][q];
-        pair_into<D, Law, PER, SOFT>(law, xi, xj, L, hL, rad_i, SOFT ? rad[q] : 0.0, fate_i,
-                                     SOFT ? (int64_t)fate[q] : 0, live, acc);
-      };
-      // a sub-brick walks every candidate once: its dense cells would
-      // overflow the per-lane queue of kept candidates and walk twice
-      if (FILTER && !a.brick_sub) {
-        auto near = [&](int32_t q) {
-          double dx[3];
+          for (int c = 0; c < D; ++c) xj[c] = pos[c][q];
+          pair_term<D, Law, PER, SOFT>(law, xi, xj, L, hL, t, rad_i, SOFT ? rad[q] : 0.0, fate_i,
+                                       SOFT ? (int64_t)fate[q] : 0);
 #pragma unroll
           for (int c = 0; c < D; ++c) {
-            dx[c] = xi[c] - pos[c][q];
-            if (PER) dx[c] = wrap_dx(dx[c], L[c], hL[c]);
-          }
-          double s2 = dx[0] * dx[0];
-          if (D > 1) s2 = s2 + dx[1] * dx[1];
-          if (D > 2) s2 = s2 + dx[2] * dx[2];
-          return s2 <= keep2 && q != li;
-        };
-        auto row_of = [&](int32_t q) {
-          const int hq = owner[q] & 0x7FFF;
-          return (int32_t)(hrow[hq] + (q - hs[hq]));
-        };
-        // pass 1: LDS indices of the candidates within reach, in walk order
-        int nq = 0;
-        walk([&](int32_t q) {
-          if (near(q)) {
-            if (nq < BRICK_LIST) lst[nq * nt + tid] = (uint16_t)q;
-            ++nq;
-          }
-        });
-        // pass 2: the pair body on those (and their rows as the stage-2
-        // list); a lane whose queue overflowed walks every candidate again
-        if (nq <= BRICK_LIST) {
-          for (int u = 0; u < nq; ++u) {
-            const int32_t q = lst[u * nt + tid];
-            body(q, true);
-            if (wl) a.wlist[(int64_t)u * a.ldl + i] = row_of(q);
-          }
-          if (wl) a.wlist_n[i] = nq;
-        } else {
-          int32_t cnt = 0;
-          walk([&](int32_t q) {
-            body(q, q != li);
-            if (wl && near(q)) {
-              if (cnt < a.wcap) a.wlist[(int64_t)cnt * a.ldl + i] = row_of(q);
-              ++cnt;
+            const double v = live ? t[c] : 0.0;
+            sum[c] = sum[c] + v;
+            if constexpr (G == 4) {
+              sum[c] = sum[c] + quad_lane<1>(v);
+              sum[c] = sum[c] + quad_lane<2>(v);
+              sum[c] = sum[c] + quad_lane<3>(v);
             }
-          });
-          if (wl) {
-            a.wlist_n[i] = cnt < a.wcap ? cnt : a.wcap;
+          }
+        };
+        if constexpr (FILTER) {
+          auto near = [&](int32_t q) {
+            double dx[3];
+#pragma unroll
+            for (int c = 0; c < D; ++c) {
+              dx[c] = xi[c] - pos[c][q];
+              if (PER) dx[c] = wrap_dx(dx[c], L[c], hL[c]);
+            }
+            double s2 = dx[0] * dx[0];
+            if (D > 1) s2 = s2 + dx[1] * dx[1];
+            if (D > 2) s2 = s2 + dx[2] * dx[2];
+            return s2 <= keep2 && q != li;
+          };
+          // the LDS indices of the agent's candidates within reach, in walk
+          // order, in its queue; a full queue is drained: the pair bodies of
+          // its entries, and their rows as the stage-2 list
+          const int ng = nt / G;
+          uint16_t* que = lst + (tid / G);      // entry u at que[u * ng]
+          int32_t cnt = 0;
+          for (;;) {
+            int32_t nq = 0;
+            if constexpr (G == 1) {
+              // room for four more between the looks at the queues
+              while (w.more()) {
+                for (int e = 0; e < 4 && w.more(); ++e) {
+                  bool live;
+                  const int32_t q = w.next(t, sub, live);
+                  if (near(q)) que[nq++ * ng] = (uint16_t)q;
+                }
+                if (__any(nq > brick_queue(G) - 4)) break;
+              }
+            } else {
+              while (w.more()) {
+                bool live;
+                const int32_t q = w.next(t, sub, live);
+                const bool in = live && near(q);
+                const uint32_t bits = (uint32_t)(__ballot(in) >> (lane & (64 - G))) & ((1u << G) - 1u);
+                if (in) que[(nq + __popc(bits & ((1u << sub) - 1u))) * ng] = (uint16_t)q;
+                nq += __popc(bits);
+                if (__any(nq > brick_queue(G) - G)) break;
+              }
+            }
+            __builtin_amdgcn_wave_barrier();   // the agent's other lanes wrote most entries
+            for (int32_t u = sub; u - sub < nq; u += G) {
+              const bool live = u < nq;
+              const int32_t q = live ? que[u * ng] : li;
+              add(q, live);
+              if (wl && live && cnt + u < a.wcap) a.wlist[(int64_t)(cnt + u) * a.ldl + row] = (int32_t)row_of(q);
+            }
+            cnt += nq;
+            if (!w.more()) break;
+          }
+          if (wl && sub == 0 && row - sd.row_off < N) {
+            a.wlist_n[row] = cnt < a.wcap ? cnt : a.wcap;
             if (cnt > a.wcap) *a.lgate = 0;
           }
+        } else {
+          while (w.more()) {
+            bool live;
+            const int32_t q = w.next(t, sub, live);
+            add(q, live && q != li);
+          }
         }
-      } else {
-        walk([&](int32_t q) { body(q, q != li); });
+      }
+      // agent k's sum to the lane that finishes it
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        if constexpr (G == 1) acc[c] = sum[c];
+        else {
+          const double v = __shfl(sum[c], ((lane - (g0 - w0)) & (64 / G - 1)) * G, 64);
+          if (own >= g0 && own < g0 + 64 / G) acc[c] = v;
+        }
       }
     }
-    stage_finish<D, Law, NOISE, true, Noise>(a, sd, sim, i, xi, acc, upre, disp2);
+    if (i >= 0) {
+      double xi[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int c = 0; c < D; ++c) xi[c] = pos[c][own_li];
+      stage_finish<D, Law, NOISE, true, Noise>(a, sd, sim, i, xi, acc, upre, disp2);
+    }
+  }
+}
+
+template <int D, class Law, int PER, int NOISE, int G, class Noise = ConstNoise>
+__device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* lds) {
+  if (a.gate && *a.gate != a.gate_run) return;
+  brick_one<D, Law, PER, NOISE, G, false, Noise>(a, lds, xcd_tile((int)blockIdx.x, (int)gridDim.x));
+}
+
+// The sub-brick launch: the listed sub-bricks in turn.  A colony's core is a
+// few of its many sub-bricks, and a block per sub-brick spent more on finding
+// out that it had nothing to do than on the core (150,001 agents at 2 per unit
+// area, 16,641 sub-bricks, 1,200 with agents: 104 us with a block for each,
+// 67 us from the list).
+template <int D, class Law, int PER, int NOISE>
+__device__ __forceinline__ void sub_brick_body(const StageArgs& a, unsigned char* lds) {
+  if (a.gate && *a.gate != a.gate_run) return;
+  const int32_t n = *a.sub_n;
+  for (int32_t k = blockIdx.x; k < n; k += gridDim.x) {
+    brick_one<D, Law, PER, NOISE, 1, true, ConstNoise>(a, lds, a.sub_list[k]);
+    __syncthreads();
   }
 }
 
@@ -1205,7 +1356,7 @@ __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* ld
 // (its row kernel walks every row).
 template <int D, class Law, int PER, int NOISE, class Noise>
 __device__ __forceinline__ void user_brick(const StageArgs& a, unsigned char* lds) {
-  if constexpr (!general_body<Law>::value) brick_body<D, Law, PER, NOISE, Noise>(a, lds);
+  if constexpr (!general_body<Law>::value) brick_body<D, Law, PER, NOISE, 1, Noise>(a, lds);
 }
 
 // An element at a 32-bit byte offset from a base that all lanes share (a

@@ -87,12 +87,13 @@ struct alignas(8) CellRange { int32_t s, e; };
 
 // LDS of one brick block: a header of int32 words, then D position arrays
 // (and radius for soft spheres) of cap doubles, int32 fate (soft spheres),
-// the halo cells' LDS offsets (H + 1) and first rows (H), the per-lane
-// queues of kept candidates, the uint16 halo cell of each staged agent and
-// the uint16 LDS index of each home row.
+// the halo cells' LDS offsets (H + 1) and first rows (H), the queues of kept
+// candidates (one per four lanes), the uint16 halo cell of each staged agent
+// and the uint16 LDS index of each home row.
 constexpr int BRICK_HDR = 16;        // int32 words: total, per-wave sums; int64 at byte 48
-constexpr int BRICK_LIST = 12;       // queue entries per lane
 constexpr int BRICK_MAX_BLOCK = 256;
+// queue entries of an agent walked by g lanes
+constexpr int brick_queue(int g) { return g == 1 ? 14 : 24; }
 constexpr int BRICK_WORDS = 6;       // brick table entry: sim, origin x, y, z, first bucket, end bucket
 constexpr double CL_LIST_GROW = 1.05;  // radius of the stage-2 lists, in units of the law's reach
 
@@ -100,12 +101,12 @@ __host__ __device__ constexpr int brick_halo_cells(int D, int bx, int by, int bz
   return (bx + 2) * (D > 1 ? by + 2 : 1) * (D > 2 ? bz + 2 : 1);
 }
 
-__host__ __device__ inline int64_t brick_lds_bytes(int D, bool soft, int cap, int H) {
+__host__ __device__ inline int64_t brick_lds_bytes(int D, bool soft, int cap, int H, int g, bool sub) {
   int64_t b = 4 * BRICK_HDR;
   b += (int64_t)8 * cap * (D + (soft ? 1 : 0));
   if (soft) b += (int64_t)4 * cap;
   b += (int64_t)4 * (2 * H + 1);
-  b += (int64_t)2 * BRICK_LIST * BRICK_MAX_BLOCK;
+  if (!sub || D > 2) b += (int64_t)2 * brick_queue(g) * (BRICK_MAX_BLOCK / g);   // sub-bricks in the plane: no filter
   b += (int64_t)4 * cap;      // owner and home_li, uint16 each
   return (b + 15) & ~(int64_t)15;
 }
@@ -123,7 +124,15 @@ struct BrickSrc {
   uint8_t* brick_skip;            // per row: left to the row-parallel kernel
   uint8_t* blk_flag;              // per row-kernel block: holds such rows
   unsigned long long* brick_over; // count of such bricks
-  int32_t sub;                    // sub-brick pass: only bricks whose rows an earlier pass left over
+  int32_t sub;                    // sub-brick pass: rows an earlier pass left over
+  // with sub-bricks: those of brick b are sub_ids[sub_first[b] ..
+  // sub_first[b + 1]); the ones with rows of a brick left over are appended
+  // to sub_list, *sub_n long (sub_brick: their table)
+  const int32_t* sub_first;
+  const int32_t* sub_ids;
+  const int32_t* sub_brick;
+  int32_t* sub_list;
+  int32_t* sub_n;
 };
 
 // LDS of one Verlet-build brick block: the header, D position arrays of cap
@@ -204,16 +213,21 @@ struct StageArgs {
   int32_t brick_cap;            // agents a brick block can stage in LDS
   // Sub-bricks (cell-linked contexts whose population can concentrate): a
   // finer brick table, each of whose bricks lies inside one brick of the
-  // main table.  After the main brick launch a second launch over it (its
-  // copy of these arguments has brick_sub = 1) takes the rows of the main
-  // bricks too dense for LDS; what it cannot stage either is left to the
-  // row-parallel kernel.  brick2 is NULL when there is no such table.
+  // main table.  The main brick launch lists those of the main bricks too
+  // dense for LDS that hold rows (sub_list, *sub_n; sub_ids from sub_first[b]
+  // on are main brick b's); a second launch works through the list, and what it cannot stage either is
+  // left to the row-parallel kernel, which clears *sub_n.  brick2 is NULL when
+  // there is no such table.
   const int32_t* brick2;
+  const int32_t* sub_first;
+  const int32_t* sub_ids;
+  int32_t* sub_list;
+  int32_t* sub_n;
   int64_t nbricks2;
   int64_t brick_lds2;
   int32_t bdim2[3];
   int32_t brick_cap2;
-  int32_t brick_sub;
+  int32_t brick_g;              // lanes per agent of the main brick launch (1 or 4)
   int32_t wcap;                 // entries per agent of wlist
   int32_t gate_run;
   int32_t fchunk;               // flattened list stage: pairs per LDS round
