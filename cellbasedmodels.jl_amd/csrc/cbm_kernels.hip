@@ -1426,10 +1426,11 @@ template <int D, int NOISE>
 static hipError_t launch_stage_dims(int nb, int law, int periodic, const StageLaunch& L, const StageArgs& a) {
   if (law == LAW_RODS) {      // 2-D, no periodic box, no noise: the host refuses the rest
     if (D != 2 || NOISE || periodic) return hipErrorInvalidValue;
+    const dim3 cells(L.grid.x * rod_lanes<NB_CELL>::value), lists(L.grid.x * rod_lanes<NB_LIST>::value);
     switch (nb) {
-      case NB_FULL: hipLaunchKernelGGL((k_rods<NB_FULL>), L.grid, L.block, 0, L.s, a); break;
-      case NB_CELL: hipLaunchKernelGGL((k_rods<NB_CELL>), L.grid, L.block, 0, L.s, a); break;
-      default: hipLaunchKernelGGL((k_rods<NB_LIST>), L.grid, L.block, 0, L.s, a); break;
+      case NB_FULL: hipLaunchKernelGGL((k_rods<NB_FULL>), cells, L.block, 0, L.s, a); break;
+      case NB_CELL: hipLaunchKernelGGL((k_rods<NB_CELL>), cells, L.block, 0, L.s, a); break;
+      default: hipLaunchKernelGGL((k_rods<NB_LIST>), lists, L.block, 0, L.s, a); break;
     }
     return hipGetLastError();
   }
