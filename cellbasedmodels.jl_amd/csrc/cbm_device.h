@@ -73,6 +73,56 @@ __device__ __forceinline__ int64_t floor_div(double a, double b) {
   return (int64_t)k;
 }
 
+// --------------------------------------------- roots and quotients in range
+// The library's sqrt and division spend half of their instructions on scaling
+// and special values.  For x in [2^-200, 2^200) its square root needs neither
+// (these are its own Newton steps, so the bits are its bits), and the root's
+// last iterate is already a reciprocal good to a few ulps: one more step gives
+// r within (1/2 + 2^-34) ulp of 1/d for the price of three operations.
+// A pair's root and quotient take 18 operations so, and 3 for the range test,
+// against 29 with a quarter-rate reciprocal among them.
+struct RootInv { double d, r; };   // sqrt(x), 1/sqrt(x)
+
+__device__ __forceinline__ RootInv root_inv(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double e = __builtin_fma(-h, g, 0.5);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(g, e, g);
+  e = __builtin_fma(-g, g, x);
+  g = __builtin_fma(e, h, g);
+  e = __builtin_fma(-g, g, x);
+  RootInv o;
+  o.d = __builtin_fma(e, h, g);
+  const double q = h + h;
+  e = __builtin_fma(-o.d, q, 1.0);
+  o.r = __builtin_fma(e, q, q);
+  return o;
+}
+
+// s/d rounded to nearest, from r = 1/d as above, for s zero or 2^-800 <= |s|
+// <= 2^800.  Both residuals are exact; after the first correction q is s/d
+// within half an ulp, so the second rounds a value within (1/2 + 2^-34) 2^-53
+// ulp of s/d.  A quotient of two 53-bit numbers lies at least 2^-54 ulp from a
+// rounding boundary, and closer than that bound only for divisors whose
+// leading 34 bits are ones, with at most four numerators each.
+__device__ __forceinline__ double quotient(double s, double d, double r) {
+  double q = s * r;
+  q = __builtin_fma(__builtin_fma(-d, q, s), r, q);
+  return __builtin_fma(__builtin_fma(-d, q, s), r, q);
+}
+
+// Range tests on the high word: a squared distance in [2^-200, 2^200), a
+// length or constant (in magnitude) in [2^-100, 2^100), a constant there or 0.
+constexpr uint32_t ROOT_LO = (1023u - 200u) << 20, ROOT_SPAN = 400u << 20;
+__device__ __forceinline__ bool root_range(double x, uint32_t span) {
+  return (uint32_t)__double2hiint(x) - ROOT_LO < span;
+}
+__device__ __forceinline__ bool plain_length(double x) {
+  return ((uint32_t)__double2hiint(x) & 0x7FFFFFFFu) - ((1023u - 100u) << 20) < (200u << 20);
+}
+__device__ __forceinline__ bool plain_constant(double x) { return x == 0.0 || plain_length(x); }
+
 // ------------------------------------------------------------- pair laws
 // Pair magnitude s(d) of the built-in agentODE bodies with their constants
 // hoisted out of the pair loop.  operator() returns whether the pair
@@ -99,6 +149,14 @@ template <> struct PairLaw<LAW_LINEAR> {
     return d > 0.0 && d < c;
   }
   __device__ __forceinline__ double reach() const { return c; }
+  // the law for d in [2^-100, 2^100): the same values (a zero's sign aside,
+  // which no sum keeps); with plain() constants every s is in quotient's range
+  __device__ __forceinline__ bool plain() const { return plain_constant(k) && plain_constant(c); }
+  __device__ __forceinline__ bool near(double d, double& s) const {
+    const double u = c - d;
+    s = k * u;
+    return u > 0.0;
+  }
 };
 
 // c = 2 r_eq, dc = f r_eq, a4 = 4 eps / (dc - c)^2:
@@ -120,6 +178,15 @@ template <> struct PairLaw<LAW_REP_ADH> {
     return d > 0.0 && d < dc;
   }
   __device__ __forceinline__ double reach() const { return dc; }
+  __device__ __forceinline__ bool plain() const {
+    return plain_constant(k) && plain_constant(c) && plain_constant(dc) && plain_constant(a4);
+  }
+  __device__ __forceinline__ bool near(double d, double& s) const {
+    const double u = c - d, v = dc - d;
+    const double rep = k * u, adh = a4 * u * v;
+    s = u > 0.0 ? rep : adh;
+    return v > 0.0;
+  }
 };
 
 // docs/src/Aggregation.md:88-98:
@@ -189,6 +256,17 @@ template <> struct PairLaw<LAW_SOFT_SPHERES> {
     const double f = f0[2 * (fi - 1) + (fj - 1)];
     s = f * (rij / d - 1) * (mu * rij / d - 1);
     return d < mu * rij && d > 0;
+  }
+  // the same with 1/d at hand, for plain d, r_ij and constants
+  __device__ __forceinline__ bool plain() const {
+    return plain_length(mu) && plain_constant(f0[0]) && plain_constant(f0[1]) && plain_constant(f0[2]) &&
+           plain_constant(f0[3]);
+  }
+  __device__ __forceinline__ bool near(double d, double r, double rij, int64_t fi, int64_t fj, double& s) const {
+    const double f = f0[2 * (fi - 1) + (fj - 1)];
+    const double m = mu * rij;
+    s = f * (quotient(rij, d, r) - 1) * (quotient(m, d, r) - 1);
+    return d < m;
   }
   __device__ __forceinline__ bool operator()(double, double& s) const { s = 0.0; return false; }
 };

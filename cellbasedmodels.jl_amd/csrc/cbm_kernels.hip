@@ -883,8 +883,15 @@ __global__ __launch_bounds__(256) void k_adjoint_step(AdjointArgs a) {
       double s2 = r[0] * r[0];
       if (D > 1) s2 += r[1] * r[1];
       if (D > 2) s2 += r[2] * r[2];
-      const double d = sqrt(s2);
-      const double id = 1.0 / d;
+      double d, id;
+      if (__any(in && !root_range(s2, ROOT_SPAN))) {
+        d = sqrt(s2);
+        id = 1.0 / d;
+      } else {
+        const RootInv q = root_inv(s2);   // NaN for the agent itself: never active
+        d = q.d;
+        id = q.r;
+      }
       double phi, dphid, dth[3];
       const bool on = law(d, id, phi, dphid, dth) && in;
       double ru = 0.0, lr = 0.0;

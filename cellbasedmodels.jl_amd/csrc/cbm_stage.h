@@ -206,22 +206,13 @@ __device__ __forceinline__ double wrap_dx(double d, double L, double hL) {
   return d > hL ? d - L : (d < -hL ? d + L : d);
 }
 
-// One neighbor at position xj: the agentODE interaction body, added to acc
-// in the reference's per-axis order.  live = false (list padding, or the
-// agent itself) leaves acc unchanged.
-template <int D, class Law, int PER, bool SOFT>
-__device__ __forceinline__ void pair_into(const Law& law, const double* xi, const double* xj, const double* L,
-                                          const double* hL, double rad_i, double rad_j, int64_t fate_i,
-                                          int64_t fate_j, bool live, double* acc) {
-  double dx[3];
-#pragma unroll
-  for (int c = 0; c < D; ++c) {
-    dx[c] = xi[c] - xj[c];
-    if (PER) dx[c] = wrap_dx(dx[c], L[c], hL[c]);
-  }
-  double s2 = dx[0] * dx[0];
-  if (D > 1) s2 = s2 + dx[1] * dx[1];
-  if (D > 2) s2 = s2 + dx[2] * dx[2];
+// The library's terms of a pair: dx, d^2 -> the term the agentODE interaction
+// body adds to the accumulator, in the reference's per-axis order; +0 for an
+// inactive pair (the accumulator starts at +0 and a sum is -0 only when both
+// terms are, so it is never -0 and adding +0 or -0 leaves it unchanged).
+template <int D, class Law, bool SOFT>
+__device__ __forceinline__ void pair_library(const Law& law, const double* dx, double s2, double rad_i, double rad_j,
+                                             int64_t fate_i, int64_t fate_j, bool live, double* t) {
   const double d = sqrt(s2);
   double s;
   bool on;
@@ -230,19 +221,101 @@ __device__ __forceinline__ void pair_into(const Law& law, const double* xi, cons
   if constexpr (SOFT) {
     // ((s dx) / d) per axis, the reference's order (softSpheres.jl:28-29)
 #pragma unroll
-    for (int c = 0; c < D; ++c) { const double v = acc[c] + (s * dx[c]) / d; acc[c] = on ? v : acc[c]; }
+    for (int c = 0; c < D; ++c) t[c] = on ? (s * dx[c]) / d : 0.0;
   } else if (Law::per_axis_division) {
 #pragma unroll
-    for (int c = 0; c < D; ++c) { const double v = acc[c] + s * (dx[c] / d); acc[c] = on ? v : acc[c]; }
+    for (int c = 0; c < D; ++c) t[c] = on ? s * (dx[c] / d) : 0.0;
   } else {
-    // F = (s/d) (x_i - x_j).  An inactive pair adds 0*dx = +-0, which
-    // leaves acc unchanged: acc starts at +0 and a sum is -0 only when
-    // both terms are, so acc is never -0.
     const double f = s / d;
     const double fe = on ? f : 0.0;
 #pragma unroll
-    for (int c = 0; c < D; ++c) acc[c] = acc[c] + fe * dx[c];
+    for (int c = 0; c < D; ++c) t[c] = fe * dx[c];
   }
+}
+
+// Laws with near(): their root and quotient in range (root_inv, quotient).
+template <class L, class = void> struct has_near { static constexpr bool value = false; };
+template <class L> struct has_near<L, decltype((void)&L::near)> { static constexpr bool value = true; };
+
+// What a law's range test lets through: nothing unless its constants do.
+template <class Law>
+__device__ __forceinline__ uint32_t law_span(const Law& law) {
+  if constexpr (has_near<Law>::value) return law.plain() ? ROOT_SPAN : 0u;
+  else return 0u;
+}
+
+// The terms of U neighbors at positions xj (+0 for one that is not live: list
+// padding, or the agent itself).  A wavefront whose pairs all lie in range
+// takes the short root and quotient, any other the library's: the same bits.
+template <int D, class Law, int PER, bool SOFT, int U>
+__device__ __forceinline__ void pair_terms(const Law& law, uint32_t span, const double* xi, const double (*xj)[3],
+                                           const double* L, const double* hL, double rad_i, const double* rad_j,
+                                           int64_t fate_i, const int64_t* fate_j, const bool* live, double (*t)[3]) {
+  double dx[U][3], s2[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      dx[u][c] = xi[c] - xj[u][c];
+      if (PER) dx[u][c] = wrap_dx(dx[u][c], L[c], hL[c]);
+    }
+    s2[u] = dx[u][0] * dx[u][0];
+    if (D > 1) s2[u] = s2[u] + dx[u][1] * dx[u][1];
+    if (D > 2) s2[u] = s2[u] + dx[u][2] * dx[u][2];
+  }
+  if constexpr (has_near<Law>::value) {
+    bool bad = false;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      bool ok = root_range(s2[u], span);
+      if constexpr (SOFT) {
+        // the numerators r_ij and s dx: no tiny offsets
+        ok = ok && plain_length(rad_i + rad_j[u]);
+#pragma unroll
+        for (int c = 0; c < D; ++c) ok = ok && plain_constant(dx[u][c]);
+      }
+      bad = bad || (live[u] && !ok);
+    }
+    if (!__any(bad)) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const RootInv q = root_inv(s2[u]);
+        double s;
+        if constexpr (SOFT) {
+          const bool on = law.near(q.d, q.r, rad_i + rad_j[u], fate_i, fate_j[u], s) && live[u];
+#pragma unroll
+          for (int c = 0; c < D; ++c) {
+            const double v = quotient(s * dx[u][c], q.d, q.r);
+            t[u][c] = on ? v : 0.0;
+          }
+        } else {
+          const bool on = law.near(q.d, s) && live[u];
+          const double f = quotient(s, q.d, q.r);
+          const double fe = on ? f : 0.0;
+#pragma unroll
+          for (int c = 0; c < D; ++c) t[u][c] = fe * dx[u][c];
+        }
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    pair_library<D, Law, SOFT>(law, dx[u], s2[u], rad_i, SOFT ? rad_j[u] : 0.0, fate_i, SOFT ? fate_j[u] : 0, live[u],
+                               t[u]);
+}
+
+// One neighbor's term.
+template <int D, class Law, int PER, bool SOFT = false>
+__device__ __forceinline__ void pair_term(const Law& law, uint32_t span, const double* xi, const double* xj,
+                                          const double* L, const double* hL, bool live, double* t, double rad_i = 0.0,
+                                          double rad_j = 0.0, int64_t fate_i = 0, int64_t fate_j = 0) {
+  double x[1][3] = {{0.0, 0.0, 0.0}}, o[1][3];
+#pragma unroll
+  for (int c = 0; c < D; ++c) x[0][c] = xj[c];
+  pair_terms<D, Law, PER, SOFT, 1>(law, span, xi, x, L, hL, rad_i, &rad_j, fate_i, &fate_j, &live, o);
+#pragma unroll
+  for (int c = 0; c < D; ++c) t[c] = o[0][c];
 }
 
 template <int D, int PER>
@@ -266,16 +339,12 @@ __device__ __forceinline__ void gather_global(const StageArgs& a, const SimDev& 
   const int64_t fate_i = SOFT ? a.fate[i] : 0;
   double L[3], hL[3];
   box_halves<D, PER>(sd, L, hL);
-  auto body = [&](const double* xj, int64_t j, bool live) {
-    pair_into<D, Law, PER, SOFT>(law, xi, xj, L, hL, rad_i, SOFT ? a.rad[j] : 0.0, fate_i,
-                                 SOFT ? a.fate[j] : 0, live, acc);
-  };
+  const uint32_t span = law_span(law);
   if (NB == NB_LIST) {
     // Verlet list in chunks of LCH gathers issued together (memory-level
     // parallelism per lane), branch-free: slots past the count read the
-    // agent itself (d = 0, never active) and add nothing.  The list
-    // indices of the next chunk are loaded before the current chunk's
-    // positions are used.
+    // agent itself and add nothing.  The list indices of the next chunk are
+    // loaded before the current chunk's positions are used.
     constexpr int LCH = CBM_LIST_CHUNK;
     const int32_t cnt = a.list_n[i];
     const int64_t ldl = a.ldl;
@@ -284,26 +353,37 @@ __device__ __forceinline__ void gather_global(const StageArgs& a, const SimDev& 
 #pragma unroll
     for (int u = 0; u < LCH; ++u) jn[u] = (u < cnt) ? lp[(int64_t)u * ldl] : (int32_t)i;
     for (int32_t q0 = 0; q0 < cnt; q0 += LCH) {
-      double px[LCH][3];
+      double px[LCH][3], t[LCH][3], rj[LCH];
       int32_t jc[LCH];
+      int64_t fj[LCH];
+      bool live[LCH];
 #pragma unroll
       for (int u = 0; u < LCH; ++u) {
         jc[u] = jn[u];
+        live[u] = q0 + u < cnt;
 #pragma unroll
         for (int c = 0; c < D; ++c) px[u][c] = a.S[c][jc[u]];
+        rj[u] = SOFT ? a.rad[jc[u]] : 0.0;
+        fj[u] = SOFT ? a.fate[jc[u]] : 0;
       }
       lp += LCH * ldl;
 #pragma unroll
       for (int u = 0; u < LCH; ++u) jn[u] = (q0 + LCH + u < cnt) ? lp[(int64_t)u * ldl] : (int32_t)i;
+      pair_terms<D, Law, PER, SOFT, LCH>(law, span, xi, px, L, hL, rad_i, rj, fate_i, fj, live, t);
 #pragma unroll
-      for (int u = 0; u < LCH; ++u) body(px[u], jc[u], q0 + u < cnt);
+      for (int u = 0; u < LCH; ++u)
+#pragma unroll
+        for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
     }
   } else {
     for_candidates<D, NB>(a, sd, N, i, [&](int64_t j) {
-      double xj[3];
+      double xj[3] = {0.0, 0.0, 0.0}, t[3];
 #pragma unroll
       for (int c = 0; c < D; ++c) xj[c] = a.S[c][j];
-      body(xj, j, true);
+      pair_term<D, Law, PER, SOFT>(law, span, xi, xj, L, hL, true, t, rad_i, SOFT ? a.rad[j] : 0.0, fate_i,
+                                   SOFT ? a.fate[j] : 0);
+#pragma unroll
+      for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[c];
     });
   }
 }
@@ -770,42 +850,6 @@ __device__ __forceinline__ void user_stage(const StageArgs& a) {
 }
 
 // ------------------------------------------------ flattened list stage
-// The pair term of one list entry: what pair_into adds to the accumulator,
-// returned instead (+0 for an inactive pair; the accumulator never holds
-// -0, so adding +0 or -0 leaves it unchanged and the sums equal pair_into's).
-template <int D, class Law, int PER, bool SOFT = false>
-__device__ __forceinline__ void pair_term(const Law& law, const double* xi, const double* xj, const double* L,
-                                          const double* hL, double* t, double rad_i = 0.0, double rad_j = 0.0,
-                                          int64_t fate_i = 0, int64_t fate_j = 0) {
-  double dx[3];
-#pragma unroll
-  for (int c = 0; c < D; ++c) {
-    dx[c] = xi[c] - xj[c];
-    if (PER) dx[c] = wrap_dx(dx[c], L[c], hL[c]);
-  }
-  double s2 = dx[0] * dx[0];
-  if (D > 1) s2 = s2 + dx[1] * dx[1];
-  if (D > 2) s2 = s2 + dx[2] * dx[2];
-  const double d = sqrt(s2);
-  double s;
-  bool on;
-  if constexpr (SOFT) on = law.pair(d, rad_i, rad_j, fate_i, fate_j, s);
-  else on = law(d, s);
-  if constexpr (SOFT) {
-    // ((s dx) / d) per axis, the reference's order (softSpheres.jl:28-29)
-#pragma unroll
-    for (int c = 0; c < D; ++c) t[c] = on ? (s * dx[c]) / d : 0.0;
-  } else if (Law::per_axis_division) {
-#pragma unroll
-    for (int c = 0; c < D; ++c) t[c] = on ? s * (dx[c] / d) : 0.0;
-  } else {
-    const double f = s / d;
-    const double fe = on ? f : 0.0;
-#pragma unroll
-    for (int c = 0; c < D; ++c) t[c] = fe * dx[c];
-  }
-}
-
 // Exclusive block scan of one int32 per thread; the total lands in *total.
 __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* wsum, int32_t* total) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = (blockDim.x + 63) >> 6;
@@ -1229,6 +1273,7 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
   // 4. the home agents
   const int32_t nh = t.r1 - t.r0;
   const Law law(sd.p);
+  const uint32_t span = law_span(law);
   double L[3], hL[3];
   box_halves<D, PER>(sd, L, hL);
   double reach2 = __builtin_inf();
@@ -1291,11 +1336,11 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
           double xj[3] = {0.0, 0.0, 0.0}, t[3];
 #pragma unroll
           for (int c = 0; c < D; ++c) xj[c] = pos[c][q];
-          pair_term<D, Law, PER, SOFT>(law, xi, xj, L, hL, t, rad_i, SOFT ? rad[q] : 0.0, fate_i,
+          pair_term<D, Law, PER, SOFT>(law, span, xi, xj, L, hL, live, t, rad_i, SOFT ? rad[q] : 0.0, fate_i,
                                        SOFT ? (int64_t)fate[q] : 0);
 #pragma unroll
           for (int c = 0; c < D; ++c) {
-            const double v = live ? t[c] : 0.0;
+            const double v = t[c];
             sum[c] = sum[c] + v;
             if constexpr (G == 4) {
               sum[c] = sum[c] + quad_lane<1>(v);
@@ -1532,12 +1577,13 @@ __device__ void clv_walk(const StageArgs& a, const SimDev& sd, int64_t i, const 
   double L[3], hL[3];
   box_halves<D, PER>(sd, L, hL);
   const double reach = law.reach();
+  const uint32_t span = law_span(law);
   double s[3] = {0.0, 0.0, 0.0};
   clv_each<D, PER>(a, sd, i, xi, reach2_bound(reach), reach + E, [&](int64_t j, double) {
     double xj[3] = {0.0, 0.0, 0.0}, t[3];
 #pragma unroll
     for (int c = 0; c < D; ++c) xj[c] = a.S[c][j];
-    pair_term<D, Law, PER>(law, xi, xj, L, hL, t);
+    pair_term<D, Law, PER>(law, span, xi, xj, L, hL, true, t);
 #pragma unroll
     for (int c = 0; c < D; ++c) s[c] = s[c] + t[c];
   });
@@ -1740,6 +1786,7 @@ __device__ __forceinline__ void clv_stage_body(const StageArgs& a, unsigned char
   const Law law(sd.p);
   double L[3], hL[3];
   box_halves<D, PER>(sd, L, hL);
+  const uint32_t span = law_span(law);
   const int32_t* __restrict__ lp = a.wlist + i;       // entry q at lp[q * ldl]
   const int64_t ldl = a.ldl;
   int32_t jn[2];
@@ -1756,14 +1803,13 @@ __device__ __forceinline__ void clv_stage_body(const StageArgs& a, unsigned char
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) jn[u] = q0 + 2 + u < n ? lp[(int64_t)(q0 + 2 + u) * ldl] : (int32_t)i;
+    const bool live[2] = {q0 < n, q0 + 1 < n};
+    double t[2][3];
+    pair_terms<D, Law, PER, false, 2>(law, span, xi, xj, L, hL, 0.0, nullptr, 0, nullptr, live, t);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      double t[3];
-      pair_term<D, Law, PER>(law, xi, xj[u], L, hL, t);
-      const bool v = q0 + u < n;
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int c = 0; c < D; ++c) acc[c] = acc[c] + (v ? t[c] : 0.0);
-    }
+      for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
   }
   double e2 = 0.0;
   stage_finish<D, Law, NOISE, true>(a, sd, ri.sim, i, xi, acc, upre, -1.0, &e2);
@@ -1852,6 +1898,7 @@ __device__ __forceinline__ void flat_body(const StageArgs& a, unsigned char* lds
   const Law law(sd.p);
   double L[3], hL[3];
   box_halves<D, PER>(sd, L, hL);
+  const uint32_t span = law_span(law);
   const int32_t* __restrict__ list = a.list;
   const int64_t ldl = a.ldl;
   double acc[3] = {0.0, 0.0, 0.0};
@@ -1885,7 +1932,7 @@ __device__ __forceinline__ void flat_body(const StageArgs& a, unsigned char* lds
         double xo[3] = {0.0, 0.0, 0.0}, t[3];
 #pragma unroll
         for (int c = 0; c < D; ++c) xo[c] = hx[c][tt[u]];
-        pair_term<D, Law, PER>(law, xo, xj[u], L, hL, t);
+        pair_term<D, Law, PER>(law, span, xo, xj[u], L, hL, true, t);
 #pragma unroll
         for (int c = 0; c < D; ++c) term[c][pp[u] - lo] = t[c];
       }
