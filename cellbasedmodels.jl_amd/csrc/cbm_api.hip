@@ -86,6 +86,8 @@ struct cbm_ctx {
   int32_t* wlist_n = nullptr;
   int32_t* fix_rows = nullptr;              // agents deferred to the exact walk, and
   int32_t* fix_n = nullptr;                 // their counts per stage
+  uint8_t* order_row = nullptr;             // rows whose list the next first stage orders, by step parity (2 C)
+  int32_t* order_ctl = nullptr;             // by step parity: the first stage orders every list
   unsigned long long* efin = nullptr;       // displacement bound and build cue since the last build
   unsigned long long* med_add = nullptr;    // a rule body's medium additions per node (32.32 fixed point)
   // the host schedules the skin-list builds of eager steps from the record
@@ -716,7 +718,7 @@ static void destroy_ctx(cbm_ctx* c) {
   for (int k = 0; k < 4 + USER_PARAMS; ++k) F(c->rule_nb[k]);
   F(c->med_init); F(c->med_tmp); F(c->adi_tab[0]); F(c->adi_tab[1]); F(c->adi_tab[2]);
   F(c->key); F(c->lin); F(c->gbucket); F(c->cell_range); F(c->count); F(c->cursor); F(c->start); F(c->tmp); F(c->cell_row);
-  F(c->emax); F(c->wlist); F(c->wlist_n); F(c->fix_rows); F(c->fix_n);
+  F(c->emax); F(c->order_row); F(c->order_ctl); F(c->wlist); F(c->wlist_n); F(c->fix_rows); F(c->fix_n);
   F(c->scan_status); F(c->scan_ticket); F(c->list); F(c->list_n); F(c->bricks); F(c->bricks2);
   F(c->sub_first); F(c->sub_ids); F(c->sub_list); F(c->brick_skip); F(c->blk_flag); F(c->flags); F(c->counters);
   for (cbm_ctx::DevBuf* b : {&c->adj_tgt, &c->adj_tbase, &c->adj_invn, &c->adj_ck, &c->adj_seg, &c->adj_lam,
@@ -952,6 +954,8 @@ static int init_ctx(cbm_ctx* c) {
     HIPCHK(c, dalloc(&c->fix_rows, c->C));
     HIPCHK(c, dalloc(&c->fix_n, 2));
     HIPCHK(c, hipMemset(c->fix_n, 0, 2 * sizeof(int32_t)));
+    HIPCHK(c, dalloc(&c->order_row, 2 * c->C));
+    HIPCHK(c, dalloc(&c->order_ctl, 2));
     HIPCHK(c, dalloc(&c->efin, 2));
     HIPCHK(c, hipMemset(c->efin, 0, 2 * sizeof(unsigned long long)));
     HIPCHK(c, hipHostMalloc((void**)&c->rec_host, sizeof(ClvRecord), hipHostMallocMapped | hipHostMallocCoherent));
@@ -1003,6 +1007,7 @@ static RebuildArgs rebuild_args(cbm_ctx* c, const int32_t* flag, int32_t* flag_c
   a.emax_clear = c->clv ? nullptr : c->emax;
   a.fix_clear = c->clv ? nullptr : c->fix_n;
   a.efin_clear = c->efin;
+  a.order_set = c->order_ctl ? c->order_ctl + (c->step & 1) : nullptr;   // the next step's first stage
   return a;
 }
 
@@ -1481,6 +1486,10 @@ static int step_once(cbm_ctx* c) {
     a.wlist = c->wlist; a.wlist_n = c->wlist_n;
     a.emax = c->emax + (s & 1);
     a.emax_next = c->emax + ((s + 1) & 1);
+    a.order_row = c->order_row + (s & 1) * c->C;
+    a.order_row_next = c->order_row + ((s + 1) & 1) * c->C;
+    a.order_now = c->order_ctl + (s & 1);
+    a.order_next = c->order_ctl + ((s + 1) & 1);
     a.clv_order = first;
     a.fix_stage = first ? 0 : 1;
     a.fix_q = queue;

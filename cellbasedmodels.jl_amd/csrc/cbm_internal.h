@@ -44,6 +44,7 @@ struct RebuildArgs {
   unsigned long long* emax_clear;   // cleared by k_keys every step (may be NULL)
   int32_t* fix_clear;               // two counters cleared by k_keys every step (may be NULL)
   unsigned long long* efin_clear;   // two words cleared by k_keys when it rebuilds (may be NULL)
+  int32_t* order_set;               // set by k_keys when it rebuilds: every list needs its order (may be NULL)
 };
 
 struct ScanArgs {

@@ -85,14 +85,17 @@ __global__ __launch_bounds__(256) void k_flat(StageArgs a) {
 // per-lane key queues, blockDim x lcap uint16), the stages over them, and
 // the exact walk of the agents they deferred
 template <int D, int LAW, int PER, int NOISE>
-__global__ __launch_bounds__(256) void k_clv(StageArgs a) {
+__global__ __launch_bounds__(256, 7) void k_clv(StageArgs a) {
   extern __shared__ unsigned char clv_lds[];
   clv_stage_body<D, PairLaw<LAW>, PER, NOISE>(a, clv_lds);
 }
 
 template <int D, int LAW, int PER, int NOISE>
 __global__ __launch_bounds__(256) void k_clv_fix(StageArgs a) {
-  if (a.tick && blockIdx.x == 0 && threadIdx.x == 0) *a.tick += 1;   // the step's last kernel
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (a.tick) *a.tick += 1;                                // the step's last kernel
+    if (a.ccell_out) *a.order_now = 0;                       // read by the step's first stage alone
+  }
   if (a.fix_n[a.fix_q] == 0) return;
   clv_fix_body<D, PairLaw<LAW>, PER, NOISE>(a);
 }
@@ -116,6 +119,7 @@ __global__ __launch_bounds__(256) void k_keys(RebuildArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (a.rebuilds) *a.rebuilds += 1;
     if (a.efin_clear) { a.efin_clear[0] = 0ull; a.efin_clear[1] = 0ull; }
+    if (a.order_set) *a.order_set = 1;
   }
   if (ri.local == 0) a.count[sd.cell_off + sd.ncells + 1] = (int32_t)(sd.n_max - st.n_tot);
   if (ri.local >= st.n_tot) return;

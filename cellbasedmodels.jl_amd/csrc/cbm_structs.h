@@ -264,6 +264,13 @@ struct StageArgs {
   // also writes rec (step_no, efin) for the host, and the final stage's
   // fix kernel advances *tick (the device step).
   unsigned long long* emax_next;
+  // which lists the first stage orders: those marked in order_row (and every
+  // list when *order_now is set); a final stage marks in order_row_next, for
+  // the next step's first stage, the rows whose order a cell change touches
+  uint8_t* order_row;
+  uint8_t* order_row_next;
+  int32_t* order_now;
+  int32_t* order_next;
   ClvRecord* rec;
   int64_t* tick;
   int64_t step_no;
