@@ -141,7 +141,7 @@ struct cbm_ctx {
   int32_t* gbucket = nullptr;             // rank_off + cell -> global bucket (cell_off + Morton rank)
   CellRange* cell_range = nullptr;        // rank_off + cell -> its rows after a rebuild
   int32_t* lin = nullptr;
-  int32_t *key = nullptr, *count = nullptr, *cursor = nullptr, *start = nullptr, *tmp = nullptr, *cell_row = nullptr;
+  int32_t *key = nullptr, *count = nullptr, *rank = nullptr, *start = nullptr, *tmp = nullptr, *cell_row = nullptr;
   unsigned long long* scan_status = nullptr;   // one status word per scan tile
   int64_t scan_tiles = 0;                      // capacity of scan_status in tiles
   unsigned int* scan_ticket = nullptr;    // [0] ticket, [1] done, [2] epoch
@@ -717,7 +717,7 @@ static void destroy_ctx(cbm_ctx* c) {
   F(c->med_c[0]); F(c->med_c[1]); F(c->med_count);
   for (int k = 0; k < 4 + USER_PARAMS; ++k) F(c->rule_nb[k]);
   F(c->med_init); F(c->med_tmp); F(c->adi_tab[0]); F(c->adi_tab[1]); F(c->adi_tab[2]);
-  F(c->key); F(c->lin); F(c->gbucket); F(c->cell_range); F(c->count); F(c->cursor); F(c->start); F(c->tmp); F(c->cell_row);
+  F(c->key); F(c->lin); F(c->gbucket); F(c->cell_range); F(c->count); F(c->rank); F(c->start); F(c->tmp); F(c->cell_row);
   F(c->emax); F(c->order_row); F(c->order_ctl); F(c->wlist); F(c->wlist_n); F(c->fix_rows); F(c->fix_n);
   F(c->scan_status); F(c->scan_ticket); F(c->list); F(c->list_n); F(c->bricks); F(c->bricks2);
   F(c->sub_first); F(c->sub_ids); F(c->sub_list); F(c->brick_skip); F(c->blk_flag); F(c->flags); F(c->counters);
@@ -915,13 +915,13 @@ static int init_ctx(cbm_ctx* c) {
   HIPCHK(c, dalloc(&c->tmp, c->C));
   HIPCHK(c, dalloc(&c->cell_row, c->C));
   HIPCHK(c, dalloc(&c->count, c->NB));
-  HIPCHK(c, dalloc(&c->cursor, c->NB));
+  HIPCHK(c, dalloc(&c->rank, c->C));
   HIPCHK(c, dalloc(&c->start, c->NB + 1));
   {
     // the largest scan: the bucket table, or the rule decisions by slot
     int64_t longest = c->NB;
     for (int s = 0; s < c->S; ++s) longest = std::max<int64_t>(longest, c->sims[s].n_max + 1);
-    c->scan_tiles = scan_blocks(longest);
+    c->scan_tiles = std::max(scan_blocks(longest), scan_blocks(std::min(longest, SCAN_SHORT)));
     HIPCHK(c, dalloc(&c->scan_status, c->scan_tiles + 1));
   }
   HIPCHK(c, dalloc(&c->scan_ticket, 4));
@@ -999,7 +999,7 @@ static RebuildArgs rebuild_args(cbm_ctx* c, const int32_t* flag, int32_t* flag_c
   a.slot = (const int32_t*)c->col[C_SLOT].cur();
   a.range = c->cell_range;
   a.nr = c->NR;
-  a.key = c->key; a.lin = c->lin; a.gbucket = c->gbucket; a.count = c->count; a.cursor = c->cursor; a.start = c->start; a.tmp = c->tmp;
+  a.key = c->key; a.lin = c->lin; a.gbucket = c->gbucket; a.count = c->count; a.rank = c->rank; a.start = c->start; a.tmp = c->tmp;
   a.cell_row = c->cell_row;
   a.dims = c->dims; a.periodic = c->m.periodic; a.full = c->full ? 1 : 0;
   a.geometric = (c->verlet || c->clv) ? 1 : 0;
@@ -1017,12 +1017,12 @@ static RebuildArgs rebuild_args(cbm_ctx* c, const int32_t* flag, int32_t* flag_c
 // current buffers); otherwise the alternate buffers become current.
 // Exclusive scan of n int32 counts (see k_scan); refuses a scan with more
 // tiles than the status array holds.
-static int run_scan(cbm_ctx* c, const int32_t* flag, int32_t* count, int32_t* cursor, int32_t* start, int64_t n) {
+static int run_scan(cbm_ctx* c, const int32_t* flag, int32_t* count, int32_t* start, int64_t n) {
   if (scan_blocks(n) > c->scan_tiles)
     return fail(c, CBM_ERR_ARG, "scan longer than its status array");
   ScanArgs s;
   std::memset(&s, 0, sizeof(s));
-  s.flag = flag; s.count = count; s.cursor = cursor; s.start = start; s.n = n;
+  s.flag = flag; s.count = count; s.start = start; s.n = n;
   s.status = c->scan_status; s.ticket = c->scan_ticket; s.done = c->scan_ticket + 1;
   s.epoch = c->scan_ticket + 2; s.nblocks = scan_blocks(n);
   HIPCHK(c, launch_scan(c->stream, s));
@@ -1048,7 +1048,7 @@ static BrickSrc brick_src(cbm_ctx* c) {
 static int rebuild_chain(cbm_ctx* c, const int32_t* flag, int32_t* flag_clear, bool tick, bool copy_back) {
   RebuildArgs a = rebuild_args(c, flag, flag_clear, tick);
   HIPCHK(c, launch_keys(c->nblocks, c->block, c->stream, a));
-  int rc = run_scan(c, flag, c->count, c->cursor, c->start, c->NB);
+  int rc = run_scan(c, flag, c->count, c->start, c->NB);
   if (rc) return rc;
   HIPCHK(c, launch_scatter(c->nblocks, c->block, c->stream, a, !c->full));
   PermuteArgs pa;
@@ -1322,7 +1322,7 @@ static RuleArgs rule_args(cbm_ctx* c, int32_t* flag) {
 }
 
 static int slot_scan(cbm_ctx* c, int32_t* in, int32_t* out, int64_t n) {
-  return run_scan(c, nullptr, in, nullptr, out, n);
+  return run_scan(c, nullptr, in, out, n);
 }
 
 // agentStepRule!: decisions by slot, their prefixes, then the effects.
@@ -1339,8 +1339,10 @@ static int rule_phase(cbm_ctx* c, int32_t* flag) {
   };
   HIPCHK(c, user ? user_launch(c->user_rule[0]) : launch_rule_decide(c->nblocks, c->block, c->stream, r));
   int rc;
-  if ((rc = slot_scan(c, c->n_add_slot, c->off_add, nm))) return rc;
-  if ((rc = slot_scan(c, c->dead_slot, c->off_dead, nm))) return rc;
+  // growth and division remove nobody and the death rule adds nobody: that
+  // table stays as it was allocated, all zero
+  if (c->m.rule != CBM_RULE_DEATH && (rc = slot_scan(c, c->n_add_slot, c->off_add, nm))) return rc;
+  if (c->m.rule != CBM_RULE_GROWTH_DIVISION && (rc = slot_scan(c, c->dead_slot, c->off_dead, nm))) return rc;
   HIPCHK(c, user ? user_launch(c->user_rule[1]) : launch_rule_apply(c->nblocks, c->block, c->stream, r));
   return CBM_OK;
 }
@@ -2425,8 +2427,9 @@ static int rebuild_in_place(cbm_ctx* c, double* const* X, const int32_t* flag,
   RebuildArgs a = rebuild_args(c, flag, nullptr, false);
   for (int d = 0; d < c->dims; ++d) a.pos[d] = X[d];
   a.dead = nullptr;
+  a.rows = 1;
   HIPCHK(c, launch_keys(c->nblocks, c->block, c->stream, a));
-  int rc = run_scan(c, flag, c->count, c->cursor, c->start, c->NB);
+  int rc = run_scan(c, flag, c->count, c->start, c->NB);
   if (rc) return rc;
   HIPCHK(c, launch_scatter(c->nblocks, c->block, c->stream, a, !c->full));
   VerletArgs va;

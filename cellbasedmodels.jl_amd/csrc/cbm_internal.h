@@ -34,9 +34,10 @@ struct RebuildArgs {
   int32_t* lin;               // per-row linear local cell
   const int32_t* gbucket;     // rank_off + linear local cell -> global bucket (cell_off + Morton rank)
   int32_t* count;             // per-bucket count
-  int32_t* cursor;            // per-bucket scatter cursor
+  int32_t* rank;              // per-row place among its bucket's rows (k_keys' order)
   int32_t* start;             // per-bucket first row (exclusive scan), nb+1 entries
-  int32_t* tmp;               // bucket-ordered source rows
+  int32_t* tmp;               // bucket-ordered slots, or source rows when rows is set
+  int32_t rows;               // the rows stay in place: the walks read them through tmp
   int32_t* cell_row;          // destination row -> linear local cell
   CellRange* range;           // rank_off + linear local cell -> rows, written by k_scatter's range blocks
   int64_t nr;                 // entries of gbucket / range (all simulations)
@@ -50,7 +51,6 @@ struct RebuildArgs {
 struct ScanArgs {
   const int32_t* flag;
   int32_t* count;
-  int32_t* cursor;
   int32_t* start;
   int64_t n;
   unsigned long long* status;
@@ -199,12 +199,18 @@ hipError_t launch_compact_slots(int nblocks, int block, hipStream_t s, const Rul
 hipError_t launch_commit_counts(hipStream_t s, const RuleArgs& a, int32_t nsims);
 
 // ------------------------------------------------------------- launchers
-// 16 Ki counts per tile: the look-back chain (one tile after another) sets
-// the scan's time, so fewer, larger tiles are faster
-constexpr int SCAN_THREADS = 1024;
+// Items per thread, and threads per tile.  Short scans take small tiles, so
+// that enough blocks share the loads; past half a million counts the
+// look-back over ever more tiles costs more and large tiles are faster.  256
+// against 1024 threads: 60001 counts 9.5 / 11.9 us, 524288 12.2 / 13.7,
+// 1048576 15.8 / 15.2, 4194305 43 / 30, 16777216 225 / 102 (event to event).
 constexpr int SCAN_ITEMS = 16;
-constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
-inline int scan_blocks(int64_t n) { return (int)((n + SCAN_TILE - 1) / SCAN_TILE); }
+constexpr int64_t SCAN_SHORT = 1 << 19;
+inline int scan_threads(int64_t n) { return n <= SCAN_SHORT ? 256 : 1024; }
+inline int scan_blocks(int64_t n) {
+  const int64_t tile = (int64_t)scan_threads(n) * SCAN_ITEMS;
+  return (int)((n + tile - 1) / tile);
+}
 
 // NB_CELL launches one block per brick (nbricks) with brick_lds bytes of LDS
 hipError_t launch_stage(int dims, int nb, int law, int nblocks, int block, hipStream_t s, const StageArgs& a,

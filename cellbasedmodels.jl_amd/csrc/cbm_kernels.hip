@@ -122,47 +122,73 @@ __global__ __launch_bounds__(256) void k_keys(RebuildArgs a) {
     if (a.order_set) *a.order_set = 1;
   }
   if (ri.local == 0) a.count[sd.cell_off + sd.ncells + 1] = (int32_t)(sd.n_max - st.n_tot);
-  if (ri.local >= st.n_tot) return;
   const int64_t r = ri.row;
-  int32_t c, lin = 0;
-  if (a.dead && a.dead[r]) c = (int32_t)(sd.cell_off + sd.ncells);
-  else if (a.full) c = (int32_t)sd.cell_off;
-  else {
-    int32_t q[3] = {0, 0, 0};
-    for (int d = 0; d < a.dims; ++d) q[d] = axis_cell(sd, d, a.pos[d][r], a.periodic, a.geometric);
-    lin = q[0] + sd.gn[0] * (q[1] + sd.gn[1] * q[2]);
-    c = a.gbucket[sd.rank_off + lin];        // cell_off + Morton rank of the cell
+  const bool live = ri.local < st.n_tot;
+  int32_t c = -1, lin = 0;
+  if (live) {
+    if (a.dead && a.dead[r]) c = (int32_t)(sd.cell_off + sd.ncells);
+    else if (a.full) c = (int32_t)sd.cell_off;
+    else {
+      int32_t q[3] = {0, 0, 0};
+      for (int d = 0; d < a.dims; ++d) q[d] = axis_cell(sd, d, a.pos[d][r], a.periodic, a.geometric);
+      lin = q[0] + sd.gn[0] * (q[1] + sd.gn[1] * q[2]);
+      c = a.gbucket[sd.rank_off + lin];        // cell_off + Morton rank of the cell
+    }
   }
+  // Runs of equal buckets along the wavefront: the first lane counts the run
+  // and its answer gives every row of it a place in the bucket.  Rows keep the
+  // last step's order, so runs are long; with one atomic per row the atomics
+  // of a cell were a serial chain, here and again in k_scatter for the places
+  // (a 165k-agent 2-D colony: 15.3 -> 6.0 us, k_scatter 20.0 -> 4.9).
+  const int lane = threadIdx.x & 63;
+  const int width = __popcll(__ballot(1));     // here, where every lane of the block takes part
+  const int32_t left = __shfl_up(c, 1, 64);
+  const unsigned long long heads = __ballot(lane == 0 || left != c);
+  const unsigned long long upto = ~0ull >> (63 - lane);      // lanes 0 .. lane
+  const int h = 63 - __clzll(heads & upto);
+  const unsigned long long later = heads & ~upto;
+  const int end = later ? __ffsll(later) - 1 : width;
+  int32_t base = 0;
+  if (h == lane && live) base = atomicAdd(&a.count[c], end - lane);
+  base = __shfl(base, h, 64);
+  if (!live) return;
   a.key[r] = c;
   a.lin[r] = lin;
-  atomicAdd(&a.count[c], 1);
+  a.rank[r] = base + (lane - h);
 }
 
 // Single-pass exclusive scan with decoupled look-back (Merrill & Garland,
 // "Single-pass Parallel Prefix Scan with Decoupled Look-back", 2016).  Tiles
 // are ordered by an atomic ticket, so a tile only ever waits on tiles that
 // are already running; status words carry a launch epoch kept in device
-// memory (so graph replays stay distinct) and never need clearing.  The scan also zeroes count[] and cursor[] for the next
+// memory (so graph replays stay distinct) and never need clearing.  A status
+// word carries the value it announces and nothing else is passed between
+// tiles, so its accesses are relaxed: an acquire in the polling loop would
+// drop the caches each time round (300k counts: 10.1 -> 7.2 us, with the
+// smaller tiles).  The scan also zeroes count[] for the next
 // rebuild.
 
 __device__ __forceinline__ unsigned long long scan_word(unsigned int epoch, unsigned int flag, unsigned int value) {
   return ((unsigned long long)(epoch & 0x3FFFFFFFu) << 34) | ((unsigned long long)flag << 32) | value;
 }
 
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan(ScanArgs a) {
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_scan(ScanArgs a) {
   if (a.flag && *a.flag == 0) return;
   __shared__ unsigned int s_tile;
-  __shared__ int32_t s_wave[SCAN_THREADS / 64];
+  __shared__ int32_t s_wave[THREADS / 64];
   __shared__ int32_t s_prefix;
   const int tid = threadIdx.x;
   __shared__ unsigned int s_epoch;
+  const bool alone = gridDim.x == 1;      // one tile needs no ticket and announces nothing
   if (tid == 0) {
-    s_tile = atomicAdd(a.ticket, 1u);
-    s_epoch = __hip_atomic_load(a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_tile = alone ? 0u : atomicAdd(a.ticket, 1u);
+    s_epoch = alone ? 0u : __hip_atomic_load(a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_prefix = 0;
   }
   __syncthreads();
   const int64_t tile = s_tile;
-  const int64_t base = tile * SCAN_TILE + (int64_t)tid * SCAN_ITEMS;
+  const int64_t base = (tile * THREADS + tid) * SCAN_ITEMS;
   // a thread's items are contiguous: whole chunks move as 16-byte vectors
   const bool whole = base + SCAN_ITEMS <= a.n;
   int32_t v[SCAN_ITEMS];
@@ -191,12 +217,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(ScanArgs a) {
   __syncthreads();
   int32_t wave_off = 0, total = 0;
 #pragma unroll
-  for (int w = 0; w < SCAN_THREADS / 64; ++w) {
+  for (int w = 0; w < THREADS / 64; ++w) {
     const int32_t t = s_wave[w];
     if (w < wave) wave_off += t;
     total += t;
   }
-  if (wave == 0) {
+  if (wave == 0 && !alone) {
     // Publish this tile's aggregate, then look back 64 tiles at a time: lane
     // l reads tile p - l; the window ends at the nearest tile that already
     // holds its inclusive prefix (tiles before 0 count as an inclusive 0).
@@ -204,13 +230,13 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(ScanArgs a) {
     int32_t prefix = 0;
     if (lane == 0)
       __hip_atomic_store(&a.status[tile], scan_word(ep, tile == 0 ? 2u : 1u, (unsigned int)total),
-                         __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int64_t p = tile - 1;
     while (p >= 0) {
       const int64_t q = p - lane;
       unsigned int fl = 2u, val = 0u;
       if (q >= 0) {
-        const unsigned long long w = __hip_atomic_load(&a.status[q], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long w = __hip_atomic_load(&a.status[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         fl = ((unsigned int)(w >> 34) == ep) ? ((unsigned int)(w >> 32) & 3u) : 0u;
         val = (unsigned int)w;
       }
@@ -229,7 +255,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(ScanArgs a) {
     if (lane == 0) {
       if (tile > 0)
         __hip_atomic_store(&a.status[tile], scan_word(ep, 2u, (unsigned int)(prefix + total)),
-                           __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       s_prefix = prefix;
     }
   }
@@ -246,7 +272,6 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(ScanArgs a) {
       q.w = run; run += v[k + 3];
       *(int4*)(a.start + base + k) = q;
       *(int4*)(a.count + base + k) = z;
-      if (a.cursor) *(int4*)(a.cursor + base + k) = z;
     }
     if (base + SCAN_ITEMS == a.n) a.start[a.n] = run;
   } else {
@@ -256,13 +281,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(ScanArgs a) {
       if (idx < a.n) {
         a.start[idx] = run;
         a.count[idx] = 0;
-        if (a.cursor) a.cursor[idx] = 0;
         run += v[k];
         if (idx == a.n - 1) a.start[a.n] = run;
       }
     }
   }
-  if (tid == 0) {
+  if (tid == 0 && !alone) {
     const unsigned int fin = atomicAdd(a.done, 1u);
     if (fin == (unsigned int)a.nblocks - 1u) {
       // every tile has read the epoch and published; advance it for the next launch
@@ -294,13 +318,35 @@ __global__ __launch_bounds__(256) void k_scatter(RebuildArgs a, int nrow) {
   const int32_t c = a.key[r];
   int32_t pos;
   if (a.full && c == (int32_t)sd.cell_off) pos = a.start[c] + a.slot[r];
-  else pos = a.start[c] + atomicAdd(&a.cursor[c], 1);
-  a.tmp[pos] = (int32_t)r;
+  else pos = a.start[c] + a.rank[r];
+  a.tmp[pos] = a.rows ? (int32_t)r : a.slot[r];
 }
 
+// Row `from` of every column of src to row `to` of dst.  Eight columns are in
+// flight: the stores of one could alias the loads of the next as far as the
+// compiler knows, and one column after the other is a chain of memory round
+// trips.
+__device__ __forceinline__ void move_row(const PermCols& cols, void* const* src, void* const* dst,
+                                         int64_t from, int64_t to) {
+  constexpr int U = 8;
+  for (int k0 = 0; k0 < cols.n; k0 += U) {
+    uint64_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k0 + u < cols.n)
+        v[u] = cols.bytes[k0 + u] == 8 ? ((const uint64_t*)src[k0 + u])[from] : ((const uint32_t*)src[k0 + u])[from];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k0 + u < cols.n) {
+        if (cols.bytes[k0 + u] == 8) ((uint64_t*)dst[k0 + u])[to] = v[u];
+        else ((uint32_t*)dst[k0 + u])[to] = (uint32_t)v[u];
+      }
+  }
+}
 
-// Each source row finds its rank by logical slot inside its bucket and
-// moves every column to that row of the alternate buffers.
+// Each source row finds its rank by logical slot inside its bucket, among
+// slots that k_scatter laid side by side, and moves every column to that row
+// of the alternate buffers.
 __global__ __launch_bounds__(256) void k_permute(PermuteArgs pa) {
   const RebuildArgs& a = pa.rb;
   if (a.flag && *a.flag == 0) return;
@@ -317,15 +363,11 @@ __global__ __launch_bounds__(256) void k_permute(PermuteArgs pa) {
   else {
     const int32_t s1 = a.start[c + 1];
     int32_t rank = 0;
-    for (int32_t q = s0; q < s1; ++q) rank += (a.slot[a.tmp[q]] < my) ? 1 : 0;
+#pragma unroll 8
+    for (int32_t q = s0; q < s1; ++q) rank += (a.tmp[q] < my) ? 1 : 0;
     dst = s0 + rank;
   }
-  for (int k = 0; k < pa.cols.n; ++k) {
-    if (pa.cols.bytes[k] == 8)
-      ((uint64_t*)pa.cols.alt[k])[dst] = ((const uint64_t*)pa.cols.cur[k])[r];
-    else
-      ((uint32_t*)pa.cols.alt[k])[dst] = ((const uint32_t*)pa.cols.cur[k])[r];
-  }
+  move_row(pa.cols, pa.cols.cur, pa.cols.alt, r, dst);
   a.cell_row[dst] = a.lin[r];
 }
 
@@ -371,12 +413,7 @@ template <int D>
 __device__ __forceinline__ int32_t verlet_row(const VerletArgs& va, const SimDev& sd, int64_t i, int2* buf, int B) {
   const RebuildArgs& a = va.rb;
   if (!va.build) {
-    for (int k = 0; k < va.cols.n; ++k) {
-      if (va.cols.bytes[k] == 8)
-        ((uint64_t*)va.cols.cur[k])[i] = ((const uint64_t*)va.cols.alt[k])[i];
-      else
-        ((uint32_t*)va.cols.cur[k])[i] = ((const uint32_t*)va.cols.alt[k])[i];
-    }
+    move_row(va.cols, va.cols.alt, va.cols.cur, i, i);
     return 0;
   }
   double xi[3] = {0.0, 0.0, 0.0};
@@ -611,12 +648,7 @@ __global__ __launch_bounds__(256) void k_verlet_brick(VerletArgs va) {
       kept = cnt < va.cap ? cnt : va.cap;
     }
     va.list_n[i] = kept;
-    for (int c = 0; c < va.cols.n; ++c) {
-      if (va.cols.bytes[c] == 8)
-        ((uint64_t*)va.cols.cur[c])[i] = ((const uint64_t*)va.cols.alt[c])[i];
-      else
-        ((uint32_t*)va.cols.cur[c])[i] = ((const uint32_t*)va.cols.alt[c])[i];
-    }
+    move_row(va.cols, va.cols.alt, va.cols.cur, i, i);
 #pragma unroll
     for (int c = 0; c < D; ++c) va.xref[c][i] = xi[c];
   }
@@ -803,7 +835,7 @@ __global__ __launch_bounds__(256) void k_rule_apply(RuleArgs a) {
 __global__ __launch_bounds__(256) void k_compact_holes(RuleArgs a) {
   const RowIdx ri = row_index(a.g);
   const SimState& st = a.g.st[ri.sim];
-  if (ri.local >= st.n_tot) return;
+  if (ri.local >= st.n_tot || st.n_remove == 0) return;
   const int64_t r = ri.row;
   if (!a.dead[r]) return;
   const int64_t Np = st.N + st.n_add - st.n_remove;
@@ -816,7 +848,7 @@ __global__ __launch_bounds__(256) void k_compact_slots(RuleArgs a) {
   const SimState& st = a.g.st[ri.sim];
   const int64_t N = st.N, A = st.n_add, R = st.n_remove;
   const int64_t Np = N + A - R;
-  if (ri.local < st.n_tot) {
+  if (ri.local < st.n_tot && R > 0) {   // without a removal every slot is below Np
     const int64_t r = ri.row;
     if (!a.dead[r]) {
       const int64_t s = a.slot[r];
@@ -1474,7 +1506,8 @@ hipError_t launch_keys(int nblocks, int block, hipStream_t s, const RebuildArgs&
 }
 
 hipError_t launch_scan(hipStream_t s, const ScanArgs& a) {
-  hipLaunchKernelGGL(k_scan, dim3(a.nblocks), dim3(SCAN_THREADS), 0, s, a);
+  if (scan_threads(a.n) == 256) hipLaunchKernelGGL(k_scan<256>, dim3(a.nblocks), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(k_scan<1024>, dim3(a.nblocks), dim3(1024), 0, s, a);
   return hipGetLastError();
 }
 
