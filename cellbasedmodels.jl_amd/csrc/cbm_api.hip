@@ -1904,6 +1904,7 @@ int cbm_compile_model(cbm_ctx* c, const char* law_body, const char* noise_body, 
       for (int v = 0; v < c->nvar; ++v)
         if (!c->gacc[v]) HIPCHK(c, dalloc(&c->gacc[v], c->C));
   }
+  HIPCHK(c, hipStreamSynchronize(nullptr));   // the fills above, for which the context's stream does not wait
   return CBM_OK;
 }
 
@@ -2191,6 +2192,9 @@ int cbm_snapshot_config(cbm_ctx* c, const int32_t* fields, int32_t nfields, int3
   }
   HIPCHK(c, dalloc(&c->snap_cnt, (int64_t)capacity * c->S));
   if (c->medium) HIPCHK(c, dalloc(&c->snap_med, (int64_t)capacity * c->med_nodes));
+  // dalloc fills on the null stream, for which the context's stream does not
+  // wait: without this the fill could land on the first snapshot
+  HIPCHK(c, hipStreamSynchronize(nullptr));
   c->snap_cap = capacity;
   return CBM_OK;
 }
