@@ -192,8 +192,10 @@ struct cbm_ctx {
   double* adi_tab[3] = {nullptr, nullptr, nullptr};
   double adi_sub = 0.0, adi_main = 0.0, adi_sup = 0.0;
 
-  // staging for transfers
+  // staging for transfers; mapped host memory for reads of up to fetch_words
   void* d_staging = nullptr;
+  uint64_t *fetch_host = nullptr, *fetch_dev = nullptr;
+  int64_t fetch_words = 0;
   // evolve!(saveEach) snapshots on the device: per field capacity x C values
   // at [k * C + row_off + slot], N per simulation, the medium, t on the host
   std::vector<int32_t> snap_fields;
@@ -734,6 +736,7 @@ static void destroy_ctx(cbm_ctx* c) {
   F(c->efin);
   F(c->med_add);
   if (c->rec_host) (void)hipHostFree(c->rec_host);
+  if (c->fetch_host) (void)hipHostFree(c->fetch_host);
   if (c->user_mod) (void)hipModuleUnload(c->user_mod);
   if (c->model_mod) (void)hipModuleUnload(c->model_mod);
   if (c->model_t) (void)hipFree(c->model_t);
@@ -967,6 +970,10 @@ static int init_ctx(cbm_ctx* c) {
   for (int s = 0; s < c->S; ++s) maxn = std::max(maxn, c->sims[s].n_max);
   c->staging_bytes = maxn * 8;
   HIPCHK(c, hipMalloc(&c->d_staging, (size_t)c->staging_bytes));
+  c->fetch_words = std::min(maxn, FETCH_MAX);
+  HIPCHK(c, hipHostMalloc((void**)&c->fetch_host, sizeof(uint64_t) * (size_t)(FETCH_HEAD + c->fetch_words),
+                          hipHostMallocMapped | hipHostMallocCoherent));
+  HIPCHK(c, hipHostGetDevicePointer((void**)&c->fetch_dev, c->fetch_host, 0));
   HIPCHK(c, hipDeviceSynchronize());
   return CBM_OK;
 }
@@ -1605,10 +1612,23 @@ static int neighbor_update(cbm_ctx* c, int64_t s, bool disp) {
   return CBM_OK;
 }
 
-static int check_flags(cbm_ctx* c) {
-  int32_t f[8];
-  HIPCHK(c, hipMemcpyAsync(f, c->flags, sizeof(f), hipMemcpyDeviceToHost, c->stream));
+// Waits for the stream with the status words, a record of rec_words and an
+// array of n words in fetch_host (record at FETCH_FLAGS, array at FETCH_HEAD).
+static int fetch(cbm_ctx* c, const void* rec, int rec_words, const void* data, int64_t n) {
+  FetchArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.flags = (const uint64_t*)c->flags;
+  a.flags_out = c->fetch_dev;
+  a.rec = (const uint64_t*)rec; a.rec_out = c->fetch_dev + FETCH_FLAGS; a.rec_n = rec_words;
+  a.data = (const uint64_t*)data; a.data_out = c->fetch_dev + FETCH_HEAD; a.n = n;
+  HIPCHK(c, launch_fetch(c->stream, a));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  return CBM_OK;
+}
+
+// The status words of the last fetch.
+static int flags_status(cbm_ctx* c) {
+  const int32_t* f = (const int32_t*)c->fetch_host;
   if (f[2]) return fail(c, CBM_ERR_LIST_OVERFLOW, "Verlet list overflow: raise nMaxNeighbors");
   if (f[3] & 2) return fail(c, CBM_ERR_CONFIG, "an agentRule body added more than 2 agents for one agent in one step");
   if (f[3] & 4) return fail(c, CBM_ERR_CONFIG, "an agentRule body looped over neighbors without naming forNeighbors");
@@ -1618,6 +1638,11 @@ static int check_flags(cbm_ctx* c) {
     return fail(c, CBM_ERR_NONFINITE, "rod contact with d_i < r_ij < (d_i + d_j)/2: the overlap d_i - r_ij is negative "
                                       "and (d_i - r_ij)^1.5 has no real value");
   return CBM_OK;
+}
+
+static int check_flags(cbm_ctx* c) {
+  const int rc = fetch(c, nullptr, 0, nullptr, 0);
+  return rc ? rc : flags_status(c);
 }
 
 // ------------------------------------------------- allocation-free counts
@@ -1978,8 +2003,13 @@ static int xfer(cbm_ctx* c, int32_t field, void* host, int64_t n, int32_t sim, b
   a.n = n;
   a.sim = sim;
   if (up) HIPCHK(c, hipMemcpyAsync(c->d_staging, host, (size_t)n * bytes, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, launch_xfer(c->nblocks, c->block, c->stream, a));
-  if (!up) {
+  const int nb = (int)((c->sims[sim].n_max + c->block - 1) / c->block);
+  HIPCHK(c, launch_xfer(nb, c->block, c->stream, a));
+  if (!up && n <= c->fetch_words) {
+    const int rc = fetch(c, nullptr, 0, c->d_staging, (n * bytes + 7) / 8);
+    if (rc) return rc;
+    std::memcpy(host, c->fetch_host + FETCH_HEAD, (size_t)n * bytes);
+  } else if (!up) {
     HIPCHK(c, hipMemcpyAsync(host, c->d_staging, (size_t)n * bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
   } else {
@@ -1996,7 +2026,7 @@ int cbm_upload(cbm_ctx* c, int32_t field, const void* host, int64_t n, int32_t s
 int cbm_download(cbm_ctx* c, int32_t field, void* host, int64_t n, int32_t sim) {
   int rc = xfer(c, field, host, n, sim, false);
   if (rc) return rc;
-  return check_flags(c);
+  return n > 0 && n <= c->fetch_words ? flags_status(c) : check_flags(c);   // a short read brought the words along
 }
 
 int cbm_set_n(cbm_ctx* c, int32_t sim, int64_t n) {
@@ -2118,19 +2148,18 @@ int cbm_sync(cbm_ctx* c) {
 
 int cbm_get_n(cbm_ctx* c, int32_t sim, int64_t* n) {
   if (!c || !n || sim < 0 || sim >= c->S) return CBM_ERR_ARG;
-  SimState st;
-  HIPCHK(c, hipMemcpyAsync(&st, c->d_st + sim, sizeof(st), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  *n = st.N;
+  static_assert(sizeof(SimState) == sizeof(uint64_t) * FETCH_REC, "one record");
+  const int rc = fetch(c, c->d_st + sim, FETCH_REC, nullptr, 0);
+  if (rc) return rc;
+  *n = ((const SimState*)(c->fetch_host + FETCH_FLAGS))->N;
   return CBM_OK;
 }
 
 int cbm_get_id_max(cbm_ctx* c, int32_t sim, int64_t* id_max) {
   if (!c || !id_max || sim < 0 || sim >= c->S) return CBM_ERR_ARG;
-  SimState st;
-  HIPCHK(c, hipMemcpyAsync(&st, c->d_st + sim, sizeof(st), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  *id_max = st.id_max;
+  const int rc = fetch(c, c->d_st + sim, FETCH_REC, nullptr, 0);
+  if (rc) return rc;
+  *id_max = ((const SimState*)(c->fetch_host + FETCH_FLAGS))->id_max;
   return CBM_OK;
 }
 
@@ -2256,14 +2285,21 @@ int cbm_snapshot_get(cbm_ctx* c, int32_t k, int32_t field, int32_t sim, void* ho
   int q = -1;
   for (size_t f = 0; f < c->snap_fields.size(); ++f) if (c->snap_fields[f] == field) q = (int)f;
   if (q < 0) return fail(c, CBM_ERR_ARG, "field not in the snapshot configuration");
-  int64_t n = 0;
-  HIPCHK(c, hipMemcpyAsync(&n, c->snap_cnt + (int64_t)k * c->S + sim, sizeof(n), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  // N, the status words and, in a short simulation, all its values at once
+  const uint64_t* src = (const uint64_t*)c->snap_buf[q] + (int64_t)k * c->C + c->h_sims[sim].row_off;
+  const int64_t n_max = c->sims[sim].n_max;
+  const bool whole = n_max <= c->fetch_words;
+  const int rc = fetch(c, c->snap_cnt + (int64_t)k * c->S + sim, 1, src, whole ? n_max : 0);
+  if (rc) return rc;
+  const int64_t n = (int64_t)c->fetch_host[FETCH_FLAGS];
   if (n_out) *n_out = n;
   if (t_out) *t_out = c->snap_t[k];
   if (n > n_cap) return fail(c, CBM_ERR_ARG, "host buffer smaller than the snapshot's N");
+  if (whole) {
+    std::memcpy(host, c->fetch_host + FETCH_HEAD, sizeof(uint64_t) * (size_t)n);
+    return flags_status(c);
+  }
   if (n > 0) {
-    const uint64_t* src = (const uint64_t*)c->snap_buf[q] + (int64_t)k * c->C + c->h_sims[sim].row_off;
     HIPCHK(c, hipMemcpyAsync(host, src, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }

@@ -95,9 +95,25 @@ struct XferArgs {
   int32_t bytes;
   int32_t to_device;
   int64_t n;            // values in staging
-  int32_t sim;          // simulation whose rows are transferred
+  int32_t sim;          // simulation whose rows are transferred (the launch has its blocks alone)
   int32_t pad;
 };
+
+// A read by the host: the status words, a record of a few words and an array
+// go to host memory mapped into the device.
+struct FetchArgs {
+  const uint64_t* flags;
+  uint64_t* flags_out;        // FETCH_FLAGS words
+  const uint64_t* rec;
+  uint64_t* rec_out;
+  const uint64_t* data;
+  uint64_t* data_out;
+  int64_t n;                  // words of data
+  int32_t rec_n;              // words of rec, at most FETCH_REC
+  int32_t pad;
+};
+constexpr int FETCH_FLAGS = 4, FETCH_REC = 8, FETCH_HEAD = 32;   // in words: flags, record, where the data begins
+constexpr int64_t FETCH_MAX = 1 << 17;                           // words a context keeps host memory for (1 MiB)
 
 // One field of every simulation gathered into slot order at
 // out[row_off + slot] (evolve!(saveEach) snapshots); n_out[sim] = N.
@@ -228,6 +244,7 @@ hipError_t launch_verlet_brick(int dims, int periodic, int64_t nbricks, int bloc
 hipError_t launch_set_flag(hipStream_t s, int32_t* flag, int32_t v);
 hipError_t launch_tick(hipStream_t s, int64_t* counter);
 hipError_t launch_xfer(int nblocks, int block, hipStream_t s, const XferArgs& a);
+hipError_t launch_fetch(hipStream_t s, const FetchArgs& a);
 hipError_t launch_snapshot(int nblocks, int block, hipStream_t s, const SnapArgs& a);
 hipError_t launch_export(int dims, int nb, int nblocks, int block, hipStream_t s, const ExportArgs& e);
 hipError_t launch_clcell(int dims, int nblocks, int block, hipStream_t s, const StageArgs& a);
