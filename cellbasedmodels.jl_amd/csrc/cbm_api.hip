@@ -2484,6 +2484,11 @@ static int rebuild_in_place(cbm_ctx* c, double* const* X, const int32_t* flag,
   va.lds_r = verlet_lds_r(c);
   va.build = 1;
   va.nopermute = 1;
+  if (c->bricks) {
+    va.bs = brick_src(c);
+    HIPCHK(c, launch_verlet_brick(c->dims, c->m.periodic, c->nbricks, c->block, c->brick_lds, c->stream, va));
+    va.fixup = 1;
+  }
   HIPCHK(c, launch_verlet(c->dims, c->nblocks, c->block, c->stream, va));
   return CBM_OK;
 }

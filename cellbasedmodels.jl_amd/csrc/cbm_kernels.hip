@@ -511,12 +511,7 @@ __device__ __forceinline__ int32_t verlet_row(const VerletArgs& va, const SimDev
     for (int32_t q = 0; q < cnt; ++q) va.list[(int64_t)q * va.ldl + i] = buf[q * B].y;
   const int32_t kept = cnt < va.cap ? cnt : va.cap;
   va.list_n[i] = kept;
-  for (int k = 0; k < (va.nopermute ? 0 : va.cols.n); ++k) {
-    if (va.cols.bytes[k] == 8)
-      ((uint64_t*)va.cols.cur[k])[i] = ((const uint64_t*)va.cols.alt[k])[i];
-    else
-      ((uint32_t*)va.cols.cur[k])[i] = ((const uint32_t*)va.cols.alt[k])[i];
-  }
+  if (!va.nopermute) move_row(va.cols, va.cols.alt, va.cols.cur, i, i);
 #pragma unroll
   for (int q = 0; q < D; ++q) va.xref[q][i] = xi[q];
   return kept;
@@ -553,7 +548,11 @@ __global__ __launch_bounds__(256) void k_verlet(VerletArgs va) {
 // registers and writes them as rows.  A list longer than the queue is rebuilt by insertion into
 // the global list, as k_verlet does past its LDS buffer, so the lists equal
 // k_verlet's.  Also copies the sorted rows back and snapshots x_ref.
-template <int D, int PER>
+// MAP: the rows stay in place and are read through the cell order's row table
+// (the adjoint's builds).  A row's walk of k_verlet loads every candidate
+// from memory through that table; here each is loaded once per brick (8 x
+// 65536 agents in 3-D: 298 -> 234 us with the pass for crowded bricks).
+template <int D, int PER, bool MAP>
 __global__ __launch_bounds__(256) void k_verlet_brick(VerletArgs va) {
   extern __shared__ unsigned char vlds[];
   const RebuildArgs& a = va.rb;
@@ -588,7 +587,8 @@ __global__ __launch_bounds__(256) void k_verlet_brick(VerletArgs va) {
   cols.xi_lds = slot;
   double unused = 0.0;
   const int b = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-  if (brick_stage<D, PER, 4, false, BX_I32>(va.bs, b, t, cols, unused) != 1) return;
+  cols.map = a.tmp;
+  if (brick_stage<D, PER, 4, false, BX_I32, MAP>(va.bs, b, t, cols, unused) != 1) return;
 
   const SimDev& sd = a.g.sims[t.sim];
   const int64_t N = a.g.st[t.sim].N;
@@ -596,7 +596,8 @@ __global__ __launch_bounds__(256) void k_verlet_brick(VerletArgs va) {
   box_halves<D, PER>(sd, L, hL);
   auto row_of = [&](int32_t q) {
     const int h = t.owner[q] & 0x7FFF;
-    return (int64_t)t.hrow[h] + (q - t.hs[h]);
+    const int64_t at = (int64_t)t.hrow[h] + (q - t.hs[h]);
+    return MAP ? (int64_t)a.tmp[at] : at;
   };
   const int32_t nh = t.r1 - t.r0;
   for (int32_t k = tid; k < nh; k += nt) {
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(256) void k_verlet_brick(VerletArgs va) {
       kept = cnt < va.cap ? cnt : va.cap;
     }
     va.list_n[i] = kept;
-    move_row(va.cols, va.cols.alt, va.cols.cur, i, i);
+    if (!MAP) move_row(va.cols, va.cols.alt, va.cols.cur, i, i);
 #pragma unroll
     for (int c = 0; c < D; ++c) va.xref[c][i] = xi[c];
   }
@@ -1543,16 +1544,22 @@ hipError_t launch_verlet(int dims, int nblocks, int block, hipStream_t s, const 
   return hipGetLastError();
 }
 
+template <int D, int PER>
+static void verlet_brick_one(dim3 g, dim3 bl, size_t lds, hipStream_t s, const VerletArgs& a) {
+  if (a.nopermute) hipLaunchKernelGGL((k_verlet_brick<D, PER, true>), g, bl, lds, s, a);
+  else hipLaunchKernelGGL((k_verlet_brick<D, PER, false>), g, bl, lds, s, a);
+}
+
 hipError_t launch_verlet_brick(int dims, int periodic, int64_t nbricks, int block, size_t lds, hipStream_t s,
                                const VerletArgs& a) {
   const dim3 g((unsigned)nbricks), bl(block);
   switch (dims * 2 + (periodic ? 1 : 0)) {
-    case 2: hipLaunchKernelGGL((k_verlet_brick<1, 0>), g, bl, lds, s, a); break;
-    case 3: hipLaunchKernelGGL((k_verlet_brick<1, 1>), g, bl, lds, s, a); break;
-    case 4: hipLaunchKernelGGL((k_verlet_brick<2, 0>), g, bl, lds, s, a); break;
-    case 5: hipLaunchKernelGGL((k_verlet_brick<2, 1>), g, bl, lds, s, a); break;
-    case 6: hipLaunchKernelGGL((k_verlet_brick<3, 0>), g, bl, lds, s, a); break;
-    default: hipLaunchKernelGGL((k_verlet_brick<3, 1>), g, bl, lds, s, a); break;
+    case 2: verlet_brick_one<1, 0>(g, bl, lds, s, a); break;
+    case 3: verlet_brick_one<1, 1>(g, bl, lds, s, a); break;
+    case 4: verlet_brick_one<2, 0>(g, bl, lds, s, a); break;
+    case 5: verlet_brick_one<2, 1>(g, bl, lds, s, a); break;
+    case 6: verlet_brick_one<3, 0>(g, bl, lds, s, a); break;
+    default: verlet_brick_one<3, 1>(g, bl, lds, s, a); break;
   }
   return hipGetLastError();
 }

@@ -948,6 +948,7 @@ struct BrickCols {
   double* xd_lds;
   const void* xi;           // integer column
   int32_t* xi_lds;
+  const int32_t* map;       // MAP: the row at each place of the cell order (rows that stay in place)
 };
 
 // Stages brick b: the rows and counts of its halo cells (wrapped on a
@@ -956,7 +957,7 @@ struct BrickCols {
 // LDS index q (halo-cell order, x fastest).  Returns 0 for an empty brick, 2
 // for one whose halo exceeds cap (its rows are then marked for the
 // row-parallel kernel), 1 when staged.
-template <int D, int PER, int U4, bool XD, int XI>
+template <int D, int PER, int U4, bool XD, int XI, bool MAP = false>
 __device__ __forceinline__ int brick_stage(const BrickSrc& src, int b, BrickTile& t, const BrickCols& cols,
                                            double& xd_max) {
   const int tid = threadIdx.x, nt = blockDim.x;
@@ -1053,6 +1054,14 @@ __device__ __forceinline__ int brick_stage(const BrickSrc& src, int b, BrickTile
     // too dense for LDS: the row-parallel kernel launched after this one
     // takes the brick's rows
     if (tid == 0 && !src.sub) atomicAdd(src.brick_over, 1ull);
+    if (MAP) {
+      for (int64_t i = (int64_t)r0 + tid; i < (int64_t)r1; i += nt) {
+        const int64_t r = cols.map[i];
+        src.brick_skip[r] = 1;
+        src.blk_flag[src.block_off[t.sim] + (r - sd.row_off) / nt] = 1;
+      }
+      return 2;
+    }
     for (int64_t i = (int64_t)r0 + tid; i < (int64_t)r1; i += nt) src.brick_skip[i] = 1;
     // wake the row-kernel blocks holding these rows (same block size)
     const int64_t q0 = src.block_off[t.sim] + ((int64_t)r0 - sd.row_off) / nt;
@@ -1098,7 +1107,8 @@ __device__ __forceinline__ int brick_stage(const BrickSrc& src, int b, BrickTile
       tag[u] = q < T ? t.owner[q] : 0;
       const int h = tag[u] & 0x7FFF;
       row[u] = q < T ? (int64_t)hrow[h] + (q - hs[h]) : -1;
-      const int64_t rr = row[u] < 0 ? (int64_t)r0 : row[u];
+      int64_t rr = row[u] < 0 ? (int64_t)r0 : row[u];
+      if (MAP) rr = cols.map[rr];
 #pragma unroll
       for (int c = 0; c < D; ++c) v[u][c] = cols.S[c][rr];
       if (XD) vd[u] = cols.xd[rr];
