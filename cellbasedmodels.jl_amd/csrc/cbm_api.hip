@@ -157,7 +157,6 @@ struct cbm_ctx {
   int bdim[3] = {1, 1, 1};
   int brick_cap = 0;                      // agents staged per brick block
   size_t brick_lds = 0;                   // its LDS bytes
-  size_t brick_lds_user = 0;              // and those of a hipRTC module's brick kernel (one lane per agent)
   int brick_g = 1;                        // lanes per agent in the cell-linked stage
   int32_t* bricks2 = nullptr;             // sub-bricks for dense regions (StageArgs::brick2)
   int32_t* sub_first = nullptr;           // main brick -> its sub-bricks (BrickSrc::sub_first, sub_ids)
@@ -505,7 +504,6 @@ static int setup_bricks(cbm_ctx* c) {
   const double per_brick = rho * (double)(1 << m), bricks = cells / (double)(1 << m);
   c->brick_g = c->rules || per_brick < BRICK_ONE_LANE || (D == 3 && bricks < BRICK_ONE_LANE_3D) ? 4 : 1;
   c->brick_lds = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]), c->brick_g);
-  c->brick_lds_user = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]), 1);
   std::vector<int32_t> tab;
   brick_table(c, bd, tab);
   c->nbricks = (int64_t)tab.size() / BRICK_WORDS;
@@ -1226,7 +1224,7 @@ static hipError_t stage_launch(cbm_ctx* c, const StageArgs& a) {
   if (c->user_nb == NB_CELL) {
     if (!c->user_brick[noise]) return hipErrorInvalidDeviceFunction;
     const hipError_t e = hipModuleLaunchKernel(c->user_brick[noise], (unsigned)c->nbricks, 1, 1, (unsigned)c->block,
-                                               1, 1, (unsigned)c->brick_lds_user, c->stream, params, nullptr);
+                                               1, 1, (unsigned)c->brick_lds, c->stream, params, nullptr);
     if (e != hipSuccess) return e;
   }
   return hipModuleLaunchKernel(f, (unsigned)c->nblocks, 1, 1, (unsigned)c->block, 1, 1, 0, c->stream, params, nullptr);
@@ -1707,7 +1705,7 @@ const char* cbm_last_error(const cbm_ctx* c) { return c ? c->err.c_str() : "null
 // The hipRTC program of cbm_compile_model: the user bodies in the skeletons
 // of a model of this dimension, neighbor walk (nb, one of NB_*) and box.
 static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth, const char* law_body,
-                               const char* noise_body, const char* rule_body, const char* medium_body) {
+                               const char* noise_body, const char* rule_body, const char* medium_body, int lanes) {
   const int dims = m.dims;
   const bool stages = law_body || noise_body;
   std::string src = "#define CBM_HIPRTC 1\n";
@@ -1752,8 +1750,8 @@ static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth
       std::snprintf(inst, sizeof(inst),
                     "extern \"C\" __global__ __launch_bounds__(256) void cbm_user_brick_%d(cbm::StageArgs a) {\n"
                     "  extern __shared__ unsigned char lds[];\n"
-                    "  cbm::user_brick<%d, cbm_law_t, %d, %d, cbm_noise_t>(a, lds);\n}\n",
-                    noise, dims, per, noise);
+                    "  cbm::user_brick<%d, cbm_law_t, %d, %d, cbm_noise_t, %d>(a, lds);\n}\n",
+                    noise, dims, per, noise, lanes);
       src += inst;
     }
   }
@@ -1796,7 +1794,7 @@ int cbm_compile_check(const cbm_model_desc* model, const char* law_body, const c
   const int nb = m.neighbors == CBM_FULL ? NB_FULL : (m.neighbors == CBM_CELL_LINKED ? NB_CELL : NB_LIST);
   const bool growth = m.rule == CBM_RULE_GROWTH_DIVISION || m.rule == CBM_RULE_CUSTOM;
   std::string lg;
-  const hiprtcResult r = user_compile(user_source(m, nb, growth, law_body, noise_body, rule_body, medium_body),
+  const hiprtcResult r = user_compile(user_source(m, nb, growth, law_body, noise_body, rule_body, medium_body, 4),
                                       nullptr, &lg);
   if (log) {
     const size_t n = std::min(lg.size(), (size_t)log_cap - 1);
@@ -1871,7 +1869,7 @@ int cbm_compile_model(cbm_ctx* c, const char* law_body, const char* noise_body, 
   std::vector<char> code;
   std::string log;
   const hiprtcResult r = user_compile(user_source(c->m, c->nb_kind, c->growth, law_body, noise_body, rule_body,
-                                                  medium_body), &code, &log);
+                                                  medium_body, c->brick_g), &code, &log);
   if (r != HIPRTC_SUCCESS) return fail(c, CBM_ERR_COMPILE, std::string("hipRTC: ") + log);
   const bool stages = law_body || noise_body;
   const int nb = c->m.law != CBM_LAW_NONE ? c->nb_kind : NB_FULL;

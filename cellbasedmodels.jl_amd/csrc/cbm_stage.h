@@ -1479,10 +1479,13 @@ __device__ __forceinline__ void sub_brick_body(const StageArgs& a, unsigned char
 }
 
 // The brick kernel of a hipRTC module: nothing for a general agentODE body
-// (its row kernel walks every row).
-template <int D, class Law, int PER, int NOISE, class Noise>
+// (its row kernel walks every row).  G as for the built-in laws: a user law
+// has no reach, so every candidate takes its pair body, and in bricks cut
+// small to fill the chip one lane per agent leaves most of a block idle
+// (27,991 agents in the plane, Heun: 13.9 -> 11.9 ms for 200 steps).
+template <int D, class Law, int PER, int NOISE, class Noise, int G>
 __device__ __forceinline__ void user_brick(const StageArgs& a, unsigned char* lds) {
-  if constexpr (!general_body<Law>::value) brick_body<D, Law, PER, NOISE, 1, Noise>(a, lds);
+  if constexpr (!general_body<Law>::value) brick_body<D, Law, PER, NOISE, G, Noise>(a, lds);
 }
 
 // An element at a 32-bit byte offset from a base that all lanes share (a

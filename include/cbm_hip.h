@@ -438,7 +438,7 @@ int cbm_get_bricks(cbm_ctx* ctx, int32_t* bdim, int32_t* cap, int64_t* nbricks,
 /* The sub-brick table of a CellLinked context with rules (no reference
  * counterpart; diagnostics as cbm_get_bricks): a finer tiling whose bricks
  * each lie inside one main brick, launched after the main bricks to stage
- * the rows of those too dense for LDS, each sub-brick sized for 32 agents
+ * the rows of those too dense for LDS, each sub-brick sized for 48 agents
  * per cell.  Zeros when the context has none. */
 int cbm_get_sub_bricks(cbm_ctx* ctx, int32_t* bdim, int32_t* cap, int64_t* nbricks);
 /* Neighbor lists of simulation `sim` in logical slots: counts[n] and
