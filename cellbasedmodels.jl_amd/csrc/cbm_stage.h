@@ -233,9 +233,12 @@ __device__ __forceinline__ void pair_library(const Law& law, const double* dx, d
   }
 }
 
-// Laws with near(): their root and quotient in range (root_inv, quotient).
-template <class L, class = void> struct has_near { static constexpr bool value = false; };
-template <class L> struct has_near<L, decltype((void)&L::near)> { static constexpr bool value = true; };
+// The built-in laws with near() and plain(): their root and quotient in range
+// (root_inv, quotient).  By type: a user's law may have members of any name.
+template <class L> struct has_near { static constexpr bool value = false; };
+template <> struct has_near<PairLaw<LAW_LINEAR>> { static constexpr bool value = true; };
+template <> struct has_near<PairLaw<LAW_REP_ADH>> { static constexpr bool value = true; };
+template <> struct has_near<PairLaw<LAW_SOFT_SPHERES>> { static constexpr bool value = true; };
 
 // What a law's range test lets through: nothing unless its constants do.
 template <class Law>
@@ -901,9 +904,12 @@ __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* wsum, int
 // path.
 
 // Reach of a built-in law: a pair can be active only when d < reach (all of
-// them also need d > 0).  Laws without it (user bodies) are not filtered.
-template <class L, class = void> struct has_reach { static constexpr bool value = false; };
-template <class L> struct has_reach<L, decltype((void)&L::reach)> { static constexpr bool value = true; };
+// them also need d > 0).  Laws without it are not filtered; user bodies never
+// are, whatever members they have.
+template <class L> struct has_reach { static constexpr bool value = false; };
+template <> struct has_reach<PairLaw<LAW_LINEAR>> { static constexpr bool value = true; };
+template <> struct has_reach<PairLaw<LAW_REP_ADH>> { static constexpr bool value = true; };
+template <> struct has_reach<PairLaw<LAW_AGGREGATION>> { static constexpr bool value = true; };
 
 // A bound on d^2 that keeps every pair with d = sqrt(d2) < reach: sqrt is
 // correctly rounded, so d < reach implies d2 < reach^2 (1 + 2^-51), and the
