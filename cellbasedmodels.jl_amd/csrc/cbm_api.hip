@@ -195,6 +195,7 @@ struct cbm_ctx {
   void* d_staging = nullptr;
   uint64_t *fetch_host = nullptr, *fetch_dev = nullptr;
   int64_t fetch_words = 0;
+  std::mutex fetch_mutex;
   // evolve!(saveEach) snapshots on the device: per field capacity x C values
   // at [k * C + row_off + slot], N per simulation, the medium, t on the host
   std::vector<int32_t> snap_fields;
@@ -1610,23 +1611,31 @@ static int neighbor_update(cbm_ctx* c, int64_t s, bool disp) {
   return CBM_OK;
 }
 
-// Waits for the stream with the status words, a record of rec_words and an
-// array of n words in fetch_host (record at FETCH_FLAGS, array at FETCH_HEAD).
-static int fetch(cbm_ctx* c, const void* rec, int rec_words, const void* data, int64_t n) {
+// The status words of a read.
+struct Flags { int32_t f[2 * FETCH_FLAGS]; };
+
+// Waits for the stream and reads the status words, a record of rec_words and
+// an array of n words; take(record, array) copies out what the caller wants.
+// The mapped memory they come through is the context's one, so a read has it
+// to itself until then: threads may read a context at the same time.
+template <class Take>
+static int fetch(cbm_ctx* c, Flags* fl, const void* rec, int rec_words, const void* data, int64_t n, Take&& take) {
   FetchArgs a;
   std::memset(&a, 0, sizeof(a));
   a.flags = (const uint64_t*)c->flags;
   a.flags_out = c->fetch_dev;
   a.rec = (const uint64_t*)rec; a.rec_out = c->fetch_dev + FETCH_FLAGS; a.rec_n = rec_words;
   a.data = (const uint64_t*)data; a.data_out = c->fetch_dev + FETCH_HEAD; a.n = n;
+  std::lock_guard<std::mutex> lock(c->fetch_mutex);
   HIPCHK(c, launch_fetch(c->stream, a));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::memcpy(fl->f, c->fetch_host, sizeof(fl->f));
+  take(c->fetch_host + FETCH_FLAGS, c->fetch_host + FETCH_HEAD);
   return CBM_OK;
 }
 
-// The status words of the last fetch.
-static int flags_status(cbm_ctx* c) {
-  const int32_t* f = (const int32_t*)c->fetch_host;
+static int flags_status(cbm_ctx* c, const Flags& fl) {
+  const int32_t* f = fl.f;
   if (f[2]) return fail(c, CBM_ERR_LIST_OVERFLOW, "Verlet list overflow: raise nMaxNeighbors");
   if (f[3] & 2) return fail(c, CBM_ERR_CONFIG, "an agentRule body added more than 2 agents for one agent in one step");
   if (f[3] & 4) return fail(c, CBM_ERR_CONFIG, "an agentRule body looped over neighbors without naming forNeighbors");
@@ -1639,8 +1648,9 @@ static int flags_status(cbm_ctx* c) {
 }
 
 static int check_flags(cbm_ctx* c) {
-  const int rc = fetch(c, nullptr, 0, nullptr, 0);
-  return rc ? rc : flags_status(c);
+  Flags fl;
+  const int rc = fetch(c, &fl, nullptr, 0, nullptr, 0, [](const uint64_t*, const uint64_t*) {});
+  return rc ? rc : flags_status(c, fl);
 }
 
 // ------------------------------------------------- allocation-free counts
@@ -1972,7 +1982,7 @@ static int field_col(cbm_ctx* c, int32_t field, int& k) {
   }
 }
 
-static int xfer(cbm_ctx* c, int32_t field, void* host, int64_t n, int32_t sim, bool up) {
+static int xfer(cbm_ctx* c, int32_t field, void* host, int64_t n, int32_t sim, bool up, Flags* fl = nullptr) {
   if (!c) return CBM_ERR_ARG;
   if (sim < 0 || sim >= c->S) return fail(c, CBM_ERR_ARG, "simulation index out of range");
   int k;
@@ -2004,9 +2014,9 @@ static int xfer(cbm_ctx* c, int32_t field, void* host, int64_t n, int32_t sim, b
   const int nb = (int)((c->sims[sim].n_max + c->block - 1) / c->block);
   HIPCHK(c, launch_xfer(nb, c->block, c->stream, a));
   if (!up && n <= c->fetch_words) {
-    const int rc = fetch(c, nullptr, 0, c->d_staging, (n * bytes + 7) / 8);
+    const int rc = fetch(c, fl, nullptr, 0, c->d_staging, (n * bytes + 7) / 8,
+                         [&](const uint64_t*, const uint64_t* v) { std::memcpy(host, v, (size_t)n * bytes); });
     if (rc) return rc;
-    std::memcpy(host, c->fetch_host + FETCH_HEAD, (size_t)n * bytes);
   } else if (!up) {
     HIPCHK(c, hipMemcpyAsync(host, c->d_staging, (size_t)n * bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -2022,9 +2032,10 @@ int cbm_upload(cbm_ctx* c, int32_t field, const void* host, int64_t n, int32_t s
 }
 
 int cbm_download(cbm_ctx* c, int32_t field, void* host, int64_t n, int32_t sim) {
-  int rc = xfer(c, field, host, n, sim, false);
+  Flags fl;
+  int rc = xfer(c, field, host, n, sim, false, &fl);
   if (rc) return rc;
-  return n > 0 && n <= c->fetch_words ? flags_status(c) : check_flags(c);   // a short read brought the words along
+  return n > 0 && n <= c->fetch_words ? flags_status(c, fl) : check_flags(c);   // a short read brought the words along
 }
 
 int cbm_set_n(cbm_ctx* c, int32_t sim, int64_t n) {
@@ -2144,20 +2155,28 @@ int cbm_sync(cbm_ctx* c) {
   return check_flags(c);
 }
 
+static int read_state(cbm_ctx* c, int32_t sim, SimState* st) {
+  static_assert(sizeof(SimState) == sizeof(uint64_t) * FETCH_REC, "one record");
+  Flags fl;
+  return fetch(c, &fl, c->d_st + sim, FETCH_REC, nullptr, 0,
+               [&](const uint64_t* rec, const uint64_t*) { std::memcpy(st, rec, sizeof(*st)); });
+}
+
 int cbm_get_n(cbm_ctx* c, int32_t sim, int64_t* n) {
   if (!c || !n || sim < 0 || sim >= c->S) return CBM_ERR_ARG;
-  static_assert(sizeof(SimState) == sizeof(uint64_t) * FETCH_REC, "one record");
-  const int rc = fetch(c, c->d_st + sim, FETCH_REC, nullptr, 0);
+  SimState st;
+  const int rc = read_state(c, sim, &st);
   if (rc) return rc;
-  *n = ((const SimState*)(c->fetch_host + FETCH_FLAGS))->N;
+  *n = st.N;
   return CBM_OK;
 }
 
 int cbm_get_id_max(cbm_ctx* c, int32_t sim, int64_t* id_max) {
   if (!c || !id_max || sim < 0 || sim >= c->S) return CBM_ERR_ARG;
-  const int rc = fetch(c, c->d_st + sim, FETCH_REC, nullptr, 0);
+  SimState st;
+  const int rc = read_state(c, sim, &st);
   if (rc) return rc;
-  *id_max = ((const SimState*)(c->fetch_host + FETCH_FLAGS))->id_max;
+  *id_max = st.id_max;
   return CBM_OK;
 }
 
@@ -2287,16 +2306,18 @@ int cbm_snapshot_get(cbm_ctx* c, int32_t k, int32_t field, int32_t sim, void* ho
   const uint64_t* src = (const uint64_t*)c->snap_buf[q] + (int64_t)k * c->C + c->h_sims[sim].row_off;
   const int64_t n_max = c->sims[sim].n_max;
   const bool whole = n_max <= c->fetch_words;
-  const int rc = fetch(c, c->snap_cnt + (int64_t)k * c->S + sim, 1, src, whole ? n_max : 0);
+  int64_t n = 0;
+  Flags fl;
+  const int rc = fetch(c, &fl, c->snap_cnt + (int64_t)k * c->S + sim, 1, src, whole ? n_max : 0,
+                       [&](const uint64_t* rec, const uint64_t* v) {
+                         n = (int64_t)rec[0];
+                         if (whole && n > 0 && n <= n_cap) std::memcpy(host, v, sizeof(uint64_t) * (size_t)n);
+                       });
   if (rc) return rc;
-  const int64_t n = (int64_t)c->fetch_host[FETCH_FLAGS];
   if (n_out) *n_out = n;
   if (t_out) *t_out = c->snap_t[k];
   if (n > n_cap) return fail(c, CBM_ERR_ARG, "host buffer smaller than the snapshot's N");
-  if (whole) {
-    std::memcpy(host, c->fetch_host + FETCH_HEAD, sizeof(uint64_t) * (size_t)n);
-    return flags_status(c);
-  }
+  if (whole) return flags_status(c, fl);
   if (n > 0) {
     HIPCHK(c, hipMemcpyAsync(host, src, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
