@@ -255,6 +255,57 @@ static hipError_t dalloc(T** p, int64_t n) {
   return e;
 }
 
+// Host memory that kernels write (mapped into the device).  Blocks outlive the
+// contexts that use them: a destroyed context hands its blocks, once its
+// stream has drained, to the next one of the device, and up to
+// HOST_POOL_BYTES of idle blocks stay mapped, so that pages a kernel has
+// written do not go back to the heap with every context.
+constexpr size_t HOST_POOL_BYTES = (size_t)64 << 20;
+struct HostPool {
+  struct Block { int device; size_t bytes; void* p; };
+  std::mutex mutex;
+  std::vector<Block> idle;
+  size_t idle_bytes = 0;
+
+  static size_t size_class(size_t bytes) {
+    size_t b = 4096;
+    while (b < bytes) b *= 2;
+    return b;
+  }
+  hipError_t get(int device, size_t bytes, void** p) {
+    const size_t b = size_class(bytes);
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      for (size_t k = 0; k < idle.size(); ++k)
+        if (idle[k].device == device && idle[k].bytes == b) {
+          *p = idle[k].p;
+          idle[k] = idle.back();
+          idle.pop_back();
+          idle_bytes -= b;
+          return hipSuccess;
+        }
+    }
+    return hipHostMalloc(p, b, hipHostMallocMapped | hipHostMallocCoherent);
+  }
+  void put(int device, size_t bytes, void* p) {
+    if (!p) return;
+    const size_t b = size_class(bytes);
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      if (idle_bytes + b <= HOST_POOL_BYTES) {
+        idle.push_back({device, b, p});
+        idle_bytes += b;
+        return;
+      }
+    }
+    (void)hipHostFree(p);
+  }
+};
+static HostPool& host_pool() {
+  static HostPool* pool = new HostPool;   // never destroyed: contexts may outlive static objects
+  return *pool;
+}
+
 static RowGeom geom(cbm_ctx* c) {
   RowGeom g;
   g.block_sim = c->d_block_sim;
@@ -706,6 +757,8 @@ static int alloc_column(cbm_ctx* c, int k, int bytes) {
   return CBM_OK;
 }
 
+static size_t fetch_bytes(const cbm_ctx* c) { return sizeof(uint64_t) * (size_t)(FETCH_HEAD + c->fetch_words); }
+
 static void destroy_ctx(cbm_ctx* c) {
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
@@ -734,8 +787,8 @@ static void destroy_ctx(cbm_ctx* c) {
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   F(c->efin);
   F(c->med_add);
-  if (c->rec_host) (void)hipHostFree(c->rec_host);
-  if (c->fetch_host) (void)hipHostFree(c->fetch_host);
+  host_pool().put(c->device, sizeof(ClvRecord), c->rec_host);
+  host_pool().put(c->device, fetch_bytes(c), c->fetch_host);
   if (c->user_mod) (void)hipModuleUnload(c->user_mod);
   if (c->model_mod) (void)hipModuleUnload(c->model_mod);
   if (c->model_t) (void)hipFree(c->model_t);
@@ -960,7 +1013,7 @@ static int init_ctx(cbm_ctx* c) {
     HIPCHK(c, dalloc(&c->order_ctl, 2));
     HIPCHK(c, dalloc(&c->efin, 2));
     HIPCHK(c, hipMemset(c->efin, 0, 2 * sizeof(unsigned long long)));
-    HIPCHK(c, hipHostMalloc((void**)&c->rec_host, sizeof(ClvRecord), hipHostMallocMapped | hipHostMallocCoherent));
+    HIPCHK(c, host_pool().get(c->device, sizeof(ClvRecord), (void**)&c->rec_host));
     std::memset(c->rec_host, 0, sizeof(ClvRecord));
     c->rec_host->step = -1;
     HIPCHK(c, hipHostGetDevicePointer((void**)&c->rec_dev, c->rec_host, 0));
@@ -970,8 +1023,7 @@ static int init_ctx(cbm_ctx* c) {
   c->staging_bytes = maxn * 8;
   HIPCHK(c, hipMalloc(&c->d_staging, (size_t)c->staging_bytes));
   c->fetch_words = std::min(maxn, FETCH_MAX);
-  HIPCHK(c, hipHostMalloc((void**)&c->fetch_host, sizeof(uint64_t) * (size_t)(FETCH_HEAD + c->fetch_words),
-                          hipHostMallocMapped | hipHostMallocCoherent));
+  HIPCHK(c, host_pool().get(c->device, fetch_bytes(c), (void**)&c->fetch_host));
   HIPCHK(c, hipHostGetDevicePointer((void**)&c->fetch_dev, c->fetch_host, 0));
   HIPCHK(c, hipDeviceSynchronize());
   return CBM_OK;
@@ -1768,10 +1820,36 @@ static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth
   return src;
 }
 
+// The headers a user-body program includes, embedded in this library, and
+// their FNV-1a sum: taken when the library is loaded and again when a compile
+// has failed, so that a message about a header's text says whether the text
+// was still whole.
+static const char* const rtc_headers[] = {cbm_rtc_cbm_device_h, cbm_rtc_cbm_structs_h, cbm_rtc_cbm_stage_h,
+                                          cbm_rtc_cbm_rule_h, cbm_rtc_cbm_medium_h, cbm_rtc_cbm_model_h};
+static uint64_t rtc_sum() {
+  uint64_t h = 0xcbf29ce484222325ull;
+  for (const char* t : rtc_headers)
+    for (; *t; ++t) h = (h ^ (unsigned char)*t) * 0x100000001b3ull;
+  return h;
+}
+static const uint64_t rtc_sum_loaded = rtc_sum();
+
+// The message of a failed compile: the first errors (a later one is often
+// their echo, and a reader of a long message sees its end), and whether the
+// embedded headers changed in memory.
+constexpr size_t RTC_MESSAGE = 3000;
+static std::string rtc_message(const std::string& log) {
+  std::string m = "hipRTC: ";
+  if (rtc_sum() != rtc_sum_loaded) m += "[the embedded kernel headers have changed in memory] ";
+  m += log.substr(0, RTC_MESSAGE);
+  if (log.size() > RTC_MESSAGE) m += "\n[" + std::to_string(log.size() - RTC_MESSAGE) + " more characters]";
+  return m;
+}
+
 // hipRTC of a user-body program for gfx950; the log on failure.
 static hiprtcResult user_compile(const std::string& src, std::vector<char>* code, std::string* log) {
-  const char* headers[] = {cbm_rtc_cbm_device_h, cbm_rtc_cbm_structs_h, cbm_rtc_cbm_stage_h, cbm_rtc_cbm_rule_h,
-                           cbm_rtc_cbm_medium_h, cbm_rtc_cbm_model_h};
+  const char* headers[6];
+  std::copy(rtc_headers, rtc_headers + 6, headers);
   const char* names[] = {"cbm_device.h", "cbm_structs.h", "cbm_stage.h", "cbm_rule.h", "cbm_medium.h", "cbm_model.h"};
   hiprtcProgram prog;
   hiprtcResult r = hiprtcCreateProgram(&prog, src.c_str(), "cbm_user_bodies.hip", 6, headers, names);
@@ -1845,7 +1923,7 @@ int cbm_compile_model_scope(cbm_ctx* c, const char* body) {
   std::vector<char> code;
   std::string log;
   if (user_compile(model_source(body), &code, &log) != HIPRTC_SUCCESS)
-    return fail(c, CBM_ERR_COMPILE, std::string("hipRTC: ") + log);
+    return fail(c, CBM_ERR_COMPILE, rtc_message(log));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   for (int s = 0; s < c->S; ++s) {
     int rc = params_from_device(c, s);
@@ -1880,7 +1958,7 @@ int cbm_compile_model(cbm_ctx* c, const char* law_body, const char* noise_body, 
   std::string log;
   const hiprtcResult r = user_compile(user_source(c->m, c->nb_kind, c->growth, law_body, noise_body, rule_body,
                                                   medium_body, c->brick_g), &code, &log);
-  if (r != HIPRTC_SUCCESS) return fail(c, CBM_ERR_COMPILE, std::string("hipRTC: ") + log);
+  if (r != HIPRTC_SUCCESS) return fail(c, CBM_ERR_COMPILE, rtc_message(log));
   const bool stages = law_body || noise_body;
   const int nb = c->m.law != CBM_LAW_NONE ? c->nb_kind : NB_FULL;
   if (c->user_mod) {
