@@ -1371,7 +1371,9 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
                                        SOFT ? (int64_t)fate[q] : 0);
 #pragma unroll
           for (int c = 0; c < D; ++c) {
-            const double v = t[c];
+            // a lane past the last candidate adds +0, whatever it read (0 times
+            // the offset of an agent that ran off to infinity is NaN)
+            const double v = live ? t[c] : 0.0;
             sum[c] = sum[c] + v;
             if constexpr (G == 4) {
               sum[c] = sum[c] + quad_lane<1>(v);
