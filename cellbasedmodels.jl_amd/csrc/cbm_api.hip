@@ -157,7 +157,7 @@ struct cbm_ctx {
   int bdim[3] = {1, 1, 1};
   int brick_cap = 0;                      // agents staged per brick block
   size_t brick_lds = 0;                   // its LDS bytes
-  int brick_g = 1;                        // lanes per agent in the cell-linked stage
+  int brick_form = BRICK_ONE;             // how the cell-linked stage walks them
   int32_t* bricks2 = nullptr;             // sub-bricks for dense regions (StageArgs::brick2)
   int32_t* sub_first = nullptr;           // main brick -> its sub-bricks (BrickSrc::sub_first, sub_ids)
   int32_t* sub_ids = nullptr;
@@ -493,27 +493,50 @@ static void brick_table(cbm_ctx* c, const int* bd, std::vector<int32_t>& tab) {
 // Elsewhere, past one block's population, m is lowered while there are fewer
 // than 256 bricks and more than 64 agents per brick.
 //
-// A brick walks its agents with one lane each when it holds about a block of
-// them, else with four (brick_one): 13-20 % more instructions, but no idle
-// lanes and shorter walks.  One against four lanes per agent, us per stage:
-// 238 agents a brick in 3,312 3-D bricks 135 / 165, 195 in 1,540 2-D bricks
-// 38 / 53, 190 in 289 2-D bricks 22 / 27; 51 in 392 2-D bricks 40 / 18, 54 in
-// 36 19 / 16, 157 soft spheres in 1,024 3-D bricks 114 / 81.  In space the
-// walk of 27 cells is the longer part, and while the bricks do not fill the
-// chip its latency counts: 232 agents in 432 bricks 59 / 46.
-constexpr double BRICK_ONE_LANE = 160.0;      // agents per brick from which a lane walks an agent
-constexpr double BRICK_ONE_LANE_3D = 1024.0;  // and, in space, the number of bricks
+// How a brick's agents are walked (brick_one).  One lane per agent where a brick
+// holds enough of them, once where few are expected in reach, with a drained
+// queue where they are many; four lanes in bricks cut smaller, where lanes
+// would stand idle, where rules add agents, and for many in reach in space
+// while the bricks do not fill the chip.  Ms per 20 to 100 steps, one lane
+// and one walk / one lane drained / four lanes:
+//   few in reach (2 to 7), RK4       agents per brick, bricks
+//     rep_adh 3-D                    66, 380      13.2 /  -   / 11.8
+//     rep_adh 2-D                    74, 430       9.4 /  9.9 /  8.9
+//     linear 2-D                     102, 300      8.4 /  8.6 /  8.2
+//     rep_adh 3-D                    137, 360     13.4 /  -   / 14.8
+//     linear 3-D                     147, 490     11.2 / 11.5 / 12.7
+//     rep_adh 2-D                    148, 340     10.4 /  -   / 10.9
+//     rep_adh 3-D                    255, 1,170   16.6 / 17.3 / 17.9
+//     rep_adh 2-D                    296, 1,010    9.7 / 10.1 / 11.8
+//   a user law, every candidate      102, 390     12.9 /  -   / 10.5
+//     evaluated, 2-D, RK4            201, 510     14.5 /  -   / 15.7
+//   many in reach, EM
+//     linear 2-D, 13 in reach        256, 400     1.64 / 1.46 / 1.34
+//     linear 2-D, 38 in reach        192, 550     2.00 / 1.86 / 2.06
+//     linear 3-D, 50 in reach        192, 760     6.25 / 4.95 / 5.13
+//     linear 3-D, 51 in reach        195, 2,050   14.9 / 11.6 / 12.7
+//     linear 3-D, 101 in reach       192, 860     14.7 / 12.8 / 12.2
+//     soft spheres 3-D, 12 in reach  157, 2,300   24.8 / 17.2 / 13.5
+constexpr double BRICK_ONE_WALK = 10.0;       // expected agents in reach up to which a lane walks once
+constexpr double BRICK_ONE_FEW = 115.0;       // agents per brick from which it does
+constexpr double BRICK_ONE_LANE = 160.0;      // agents per brick from which a lane walks an agent otherwise
+constexpr double BRICK_DRAIN_3D = 1024.0;     // and bricks in space
+
+static double law_reach(int law, const double* p);
 
 static int setup_bricks(cbm_ctx* c) {
   const int D = c->dims;
   const bool soft = c->inertial;
-  double rho = 0.0, agents = 0.0, cells = 0.0;
+  double rho = 0.0, agents = 0.0, cells = 0.0, in_reach = 0.0;
   for (int s = 0; s < c->S; ++s) {
     const double n = (double)std::max<int64_t>(c->rules ? c->sims[s].n_max : c->sims[s].n, 1);
     const SimDev& sd = c->h_sims[s];
     double inner = 1.0;                 // cells of the box itself
     for (int a = 0; a < D; ++a) inner *= std::max(1.0, std::min((double)sd.gn[a], sd.L[a] / sd.gedge[a]));
     rho = std::max(rho, n / inner);
+    double ball = D == 1 ? 2.0 : (D == 2 ? M_PI : 4.0 / 3.0 * M_PI);      // in cells; no law reaches past one
+    for (int a = 0; a < D; ++a) ball *= std::max(0.0, std::min(1.0, law_reach(c->m.law, c->sims[s].p) / sd.gedge[a]));
+    in_reach = std::max(in_reach, n / inner * ball);
     agents += n;
     cells += (double)sd.ncells;
   }
@@ -530,8 +553,8 @@ static int setup_bricks(cbm_ctx* c) {
   // and fate for soft spheres); both add an owner and a home-row index
   const bool build = c->verlet || c->clv;   // the bricks serve the list build
   const int64_t per = build ? 8 * D + 4 + 4 : 8 * (D + (soft ? 1 : 0)) + (soft ? 4 : 0) + 4;
-  auto tile_bytes = [&](int cp, int H, int g = 4, bool sub = false) {
-    return build ? vbrick_lds_bytes(D, cp, H) : brick_lds_bytes(D, soft, cp, H, g, sub);
+  auto tile_bytes = [&](int cp, int H, int form = BRICK_FOUR, bool sub = false) {
+    return build ? vbrick_lds_bytes(D, cp, H) : brick_lds_bytes(D, soft, cp, H, form, sub);
   };
   int bd[3] = {1, 1, 1};
   int cap = 0;
@@ -554,8 +577,13 @@ static int setup_bricks(cbm_ctx* c) {
   for (int a = 0; a < 3; ++a) c->bdim[a] = bd[a];
   c->brick_cap = cap;
   const double per_brick = rho * (double)(1 << m), bricks = cells / (double)(1 << m);
-  c->brick_g = c->rules || per_brick < BRICK_ONE_LANE || (D == 3 && bricks < BRICK_ONE_LANE_3D) ? 4 : 1;
-  c->brick_lds = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]), c->brick_g);
+  const bool user = c->m.law == CBM_LAW_CUSTOM, few = !user && in_reach <= BRICK_ONE_WALK;
+  c->brick_form = BRICK_FOUR;
+  if (!c->rules && per_brick >= (few ? BRICK_ONE_FEW : BRICK_ONE_LANE)) {
+    if (few || user) c->brick_form = BRICK_ONE;
+    else if (D < 3 || bricks >= BRICK_DRAIN_3D) c->brick_form = BRICK_DRAIN;
+  }
+  c->brick_lds = (size_t)tile_bytes(cap, brick_halo_cells(D, bd[0], bd[1], bd[2]), c->brick_form);
   std::vector<int32_t> tab;
   brick_table(c, bd, tab);
   c->nbricks = (int64_t)tab.size() / BRICK_WORDS;
@@ -573,12 +601,12 @@ static int setup_bricks(cbm_ctx* c) {
       int b2[3];
       edges(m2, b2);
       const int H2 = brick_halo_cells(D, b2[0], b2[1], b2[2]);
-      const int64_t capmax = (budget2 - tile_bytes(0, H2, 1, true) - 16) / per;
+      const int64_t capmax = (budget2 - tile_bytes(0, H2, BRICK_DRAIN, true) - 16) / per;
       const double want = 1.2 * SUB_BRICK_DENSITY * H2 + 32.0;
       if (want > (double)capmax) continue;
       for (int a = 0; a < 3; ++a) c->bdim2[a] = b2[a];
       c->brick_cap2 = (int)std::min<int64_t>(capmax, (int64_t)std::max(256.0, want));
-      c->brick_lds2 = (size_t)tile_bytes(c->brick_cap2, H2, 1, true);
+      c->brick_lds2 = (size_t)tile_bytes(c->brick_cap2, H2, BRICK_DRAIN, true);
       std::vector<int32_t> tab2;
       brick_table(c, b2, tab2);
       c->nbricks2 = (int64_t)tab2.size() / BRICK_WORDS;
@@ -1184,7 +1212,7 @@ static StageArgs stage_base(cbm_ctx* c) {
   a.brick_over = (unsigned long long*)(c->counters + 2);
   for (int q = 0; q < 3; ++q) a.bdim[q] = c->bdim[q];
   a.brick_cap = c->brick_cap;
-  a.brick_g = c->brick_g;
+  a.brick_form = c->brick_form;
   a.sub_first = c->sub_first; a.sub_ids = c->sub_ids;
   a.sub_list = c->sub_list; a.sub_n = c->sub_list ? c->sub_list + c->nbricks2 : nullptr;
   a.brick2 = c->bricks2; a.nbricks2 = c->nbricks2; a.brick_lds2 = (int64_t)c->brick_lds2;
@@ -1765,9 +1793,10 @@ const char* cbm_last_error(const cbm_ctx* c) { return c ? c->err.c_str() : "null
 }  // extern "C"
 
 // The hipRTC program of cbm_compile_model: the user bodies in the skeletons
-// of a model of this dimension, neighbor walk (nb, one of NB_*) and box.
+// of a model of this dimension, neighbor walk (nb, one of NB_*) and box and
+// the context's form of brick walk.
 static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth, const char* law_body,
-                               const char* noise_body, const char* rule_body, const char* medium_body, int lanes) {
+                               const char* noise_body, const char* rule_body, const char* medium_body, int form) {
   const int dims = m.dims;
   const bool stages = law_body || noise_body;
   std::string src = "#define CBM_HIPRTC 1\n";
@@ -1813,7 +1842,7 @@ static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth
                     "extern \"C\" __global__ __launch_bounds__(256) void cbm_user_brick_%d(cbm::StageArgs a) {\n"
                     "  extern __shared__ unsigned char lds[];\n"
                     "  cbm::user_brick<%d, cbm_law_t, %d, %d, cbm_noise_t, %d>(a, lds);\n}\n",
-                    noise, dims, per, noise, lanes);
+                    noise, dims, per, noise, form);
       src += inst;
     }
   }
@@ -1882,7 +1911,7 @@ int cbm_compile_check(const cbm_model_desc* model, const char* law_body, const c
   const int nb = m.neighbors == CBM_FULL ? NB_FULL : (m.neighbors == CBM_CELL_LINKED ? NB_CELL : NB_LIST);
   const bool growth = m.rule == CBM_RULE_GROWTH_DIVISION || m.rule == CBM_RULE_CUSTOM;
   std::string lg;
-  const hiprtcResult r = user_compile(user_source(m, nb, growth, law_body, noise_body, rule_body, medium_body, 4),
+  const hiprtcResult r = user_compile(user_source(m, nb, growth, law_body, noise_body, rule_body, medium_body, BRICK_FOUR),
                                       nullptr, &lg);
   if (log) {
     const size_t n = std::min(lg.size(), (size_t)log_cap - 1);
@@ -1957,7 +1986,7 @@ int cbm_compile_model(cbm_ctx* c, const char* law_body, const char* noise_body, 
   std::vector<char> code;
   std::string log;
   const hiprtcResult r = user_compile(user_source(c->m, c->nb_kind, c->growth, law_body, noise_body, rule_body,
-                                                  medium_body, c->brick_g), &code, &log);
+                                                  medium_body, c->brick_form), &code, &log);
   if (r != HIPRTC_SUCCESS) return fail(c, CBM_ERR_COMPILE, rtc_message(log));
   const bool stages = law_body || noise_body;
   const int nb = c->m.law != CBM_LAW_NONE ? c->nb_kind : NB_FULL;

@@ -60,11 +60,11 @@ __global__ __launch_bounds__(256) void k_rods(StageArgs a) {
 }
 
 // cell-linked stage on LDS brick tiles (dynamic LDS: brick_lds_bytes)
-// G lanes per agent; at most 128 registers, so that four blocks share a CU
-template <int D, int LAW, int PER, int NOISE, int G>
+// at most 128 registers, so that four blocks share a CU
+template <int D, int LAW, int PER, int NOISE, int FORM>
 __global__ __launch_bounds__(256, 4) void k_brick(StageArgs a) {
   extern __shared__ unsigned char brick_lds[];
-  brick_body<D, PairLaw<LAW>, PER, NOISE, G>(a, brick_lds);
+  brick_body<D, PairLaw<LAW>, PER, NOISE, FORM>(a, brick_lds);
 }
 
 template <int D, int LAW, int PER, int NOISE>
@@ -1380,13 +1380,13 @@ __global__ __launch_bounds__(256) void k_clcell(StageArgs a) {
 // ------------------------------------------------------------- launchers
 struct StageLaunch { dim3 grid, bgrid, block; size_t lds; hipStream_t s; };   // bgrid: one block per brick
 
-template <int D, int PER, int NOISE, int G>
+template <int D, int PER, int NOISE, int FORM>
 static hipError_t launch_brick(int law, dim3 grid, dim3 block, size_t lds, hipStream_t s, const StageArgs& a) {
   switch (law) {
-    case LAW_LINEAR: hipLaunchKernelGGL((k_brick<D, LAW_LINEAR, PER, NOISE, G>), grid, block, lds, s, a); break;
-    case LAW_REP_ADH: hipLaunchKernelGGL((k_brick<D, LAW_REP_ADH, PER, NOISE, G>), grid, block, lds, s, a); break;
-    case LAW_AGGREGATION: hipLaunchKernelGGL((k_brick<D, LAW_AGGREGATION, PER, NOISE, G>), grid, block, lds, s, a); break;
-    case LAW_SOFT_SPHERES: hipLaunchKernelGGL((k_brick<D, LAW_SOFT_SPHERES, PER, NOISE, G>), grid, block, lds, s, a); break;
+    case LAW_LINEAR: hipLaunchKernelGGL((k_brick<D, LAW_LINEAR, PER, NOISE, FORM>), grid, block, lds, s, a); break;
+    case LAW_REP_ADH: hipLaunchKernelGGL((k_brick<D, LAW_REP_ADH, PER, NOISE, FORM>), grid, block, lds, s, a); break;
+    case LAW_AGGREGATION: hipLaunchKernelGGL((k_brick<D, LAW_AGGREGATION, PER, NOISE, FORM>), grid, block, lds, s, a); break;
+    case LAW_SOFT_SPHERES: hipLaunchKernelGGL((k_brick<D, LAW_SOFT_SPHERES, PER, NOISE, FORM>), grid, block, lds, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1396,8 +1396,9 @@ template <int D, int NB, int PER, int NOISE>
 static hipError_t launch_stage_law(int law, const StageLaunch& L, const StageArgs& a) {
   if (NB == NB_CELL) {
     // bricks that fit in LDS, then the rows of those that did not
-    hipError_t e = a.brick_g == 1 ? launch_brick<D, PER, NOISE, 1>(law, L.bgrid, L.block, L.lds, L.s, a)
-                                  : launch_brick<D, PER, NOISE, 4>(law, L.bgrid, L.block, L.lds, L.s, a);
+    hipError_t e = a.brick_form == BRICK_ONE ? launch_brick<D, PER, NOISE, BRICK_ONE>(law, L.bgrid, L.block, L.lds, L.s, a)
+                 : a.brick_form == BRICK_DRAIN ? launch_brick<D, PER, NOISE, BRICK_DRAIN>(law, L.bgrid, L.block, L.lds, L.s, a)
+                                               : launch_brick<D, PER, NOISE, BRICK_FOUR>(law, L.bgrid, L.block, L.lds, L.s, a);
     if (e != hipSuccess) return e;
     if (a.brick2 && a.nbricks2 > 0) {
       // the sub-bricks of the bricks that did not fit, from the list

@@ -1226,21 +1226,32 @@ struct BrickWalk {
 // The cell-linked stage of a brick.  Built-in laws filter the candidates: a
 // cheap test queues the LDS indices of the pairs within the law's reach (in
 // walk order), and the full pair body runs on those only.  Every pair left
-// out is inactive, so the sum is unchanged.  A full queue is drained and
-// refilled, so cells of any density are tested once; a queue that could only
-// overflow made its lane walk all candidates again with the full body, which
-// soft spheres (15 of 132 candidates near enough, 12 queue entries) did in
-// every wavefront: 172 us per stage for 120,001 of them, 81 us now.
+// out is inactive, so the sum is unchanged.
 //
-// G lanes share an agent: they test G consecutive candidates at once and
-// evaluate G queued pairs at once, whose terms the first lane adds in order
-// (DPP moves), so the sums keep the reference's order.  With four, a
+// BRICK_ONE: a lane per agent walks once, and walks again for what its queue
+// did not hold.  That is the shortest code for the usual handful of agents in
+// reach (rep_adh in space, 4 of 27: 300,001 agents in a periodic box, RK4,
+// 50 steps 16.6 ms, with the queue drained as it fills 17.3), but where the
+// queue overflows in every wavefront the second walk costs as much as the
+// first (50 in reach, 100,001 agents: 6.3 ms against 4.9).
+//
+// BRICK_DRAIN: a lane per agent; the queue is drained and refilled, so cells of
+// any density are tested once.
+//
+// BRICK_FOUR: four lanes share an agent: they test four consecutive candidates
+// at once and evaluate four queued pairs at once, whose terms the first lane
+// adds in order (DPP moves), so the sums keep the reference's order.  A
 // wavefront waits for the longest walk of 16 agents and not of 64, bricks of
 // fewer agents than lanes keep the lanes busy, and neighboring lanes read
-// neighboring LDS words; the moves and shared adds cost instructions, so
-// bricks that fill their lanes by themselves use one (setup_bricks).
-template <int D, class Law, int PER, int NOISE, int G, bool SUB, class Noise>
+// neighboring LDS words; the moves and shared adds cost instructions.  The
+// queue is drained as it fills (soft spheres, 15 of 132 candidates near
+// enough: 172 us per stage for 120,001 of them with one lane and a second walk
+// with the full body, 81 us so).
+//
+// setup_bricks says which bricks take which.
+template <int D, class Law, int PER, int NOISE, int FORM, bool SUB, class Noise>
 __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds, int b) {
+  constexpr int G = brick_lanes(FORM);
   constexpr bool SOFT = same_type<Law, PairLaw<LAW_SOFT_SPHERES>>::value;
   // on sub-bricks in the plane every candidate takes the pair body: a third
   // of them is in reach, and the filter costs as much as it saves
@@ -1276,7 +1287,7 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
   t.hrow = (int32_t*)p;
   p += (size_t)4 * H;
   uint16_t* lst = (uint16_t*)p;       // the agents' queues of kept candidates
-  if (FILTER) p += (size_t)2 * brick_queue(G) * (BRICK_MAX_BLOCK / G);
+  if (FILTER) p += (size_t)2 * brick_queue(FORM) * (BRICK_MAX_BLOCK / G);
   t.owner = (uint16_t*)p;
   p += (size_t)2 * cap;
   t.home_li = (uint16_t*)p;
@@ -1329,7 +1340,8 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
   const int lane = tid & 63, sub = lane & (G - 1), wv = tid >> 6, nw = nt >> 6;
   for (int32_t k0 = 0; k0 < nh; k0 += nt) {
     const int32_t m = nh - k0 < nt ? nh - k0 : nt;
-    const int32_t npw = (m + nw - 1) / nw;            // agents per wavefront
+    // agents per wavefront: whole rounds of 64 / G
+    const int32_t npw = ((m + nw - 1) / nw + 64 / G - 1) & ~(64 / G - 1);
     const int32_t w0 = k0 + wv * npw;
     const int32_t w1 = w0 + npw < k0 + m ? w0 + npw : k0 + m;
     const int32_t own = w0 + lane;
@@ -1360,7 +1372,6 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
         const int64_t fate_i = SOFT ? fate[li] : 0;
         double keep2 = reach2;
         if constexpr (SOFT) keep2 = law.mu >= 0.0 ? reach2_bound(law.mu * (rad_i + rmax)) : __builtin_inf();
-        BrickWalk<D, G> w(t, h, sub);
         // G candidates' terms (this lane's is q's, nothing unless live) added
         // to the agent's sum, in their order, by its first lane
         auto add = [&](int32_t q, bool live) {
@@ -1395,50 +1406,82 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
             if (D > 2) s2 = s2 + dx[2] * dx[2];
             return s2 <= keep2 && q != li;
           };
-          // the LDS indices of the agent's candidates within reach, in walk
-          // order, in its queue; a full queue is drained: the pair bodies of
-          // its entries, and their rows as the stage-2 list
           const int ng = nt / G;
           uint16_t* que = lst + (tid / G);      // entry u at que[u * ng]
           int32_t cnt = 0;
-          for (;;) {
-            int32_t nq = 0;
-            if constexpr (G == 1) {
-              // room for four more between the looks at the queues
-              while (w.more()) {
-                for (int e = 0; e < 4 && w.more(); ++e) {
+          auto keep = [&](int32_t u, int32_t q) {      // candidate u as an entry of the stage-2 list
+            if (wl && u < a.wcap) a.wlist[(int64_t)u * a.ldl + row] = (int32_t)row_of(q);
+          };
+          if constexpr (FORM == BRICK_ONE) {
+            // one walk fills the queue, and only a lane whose queue was too
+            // short walks again for the candidates past it
+            brick_walk<D>(t, h, [&](int32_t q) {
+              if (near(q)) {
+                if (cnt < brick_queue(FORM)) que[cnt * ng] = (uint16_t)q;
+                ++cnt;
+              }
+            });
+            const int32_t nq = cnt < brick_queue(FORM) ? cnt : brick_queue(FORM);
+            for (int32_t u = 0; u < nq; ++u) {
+              const int32_t q = que[u * ng];
+              add(q, true);
+              keep(u, q);
+            }
+            if (cnt > nq) {
+              int32_t u = 0;
+              brick_walk<D>(t, h, [&](int32_t q) {
+                if (!near(q)) return;
+                if (u >= nq) { add(q, true); keep(u, q); }
+                ++u;
+              });
+            }
+          } else {
+            // the LDS indices of the agent's candidates within reach, in walk
+            // order, in its queue; a full queue is drained: the pair bodies of
+            // its entries, and their rows as the stage-2 list
+            BrickWalk<D, G> w(t, h, sub);
+            for (;;) {
+              int32_t nq = 0;
+              if constexpr (G == 1) {
+                // room for four more between the looks at the queues
+                while (w.more()) {
+                  for (int e = 0; e < 4 && w.more(); ++e) {
+                    bool live;
+                    const int32_t q = w.next(t, sub, live);
+                    if (near(q)) que[nq++ * ng] = (uint16_t)q;
+                  }
+                  if (__any(nq > brick_queue(FORM) - 4)) break;
+                }
+              } else {
+                while (w.more()) {
                   bool live;
                   const int32_t q = w.next(t, sub, live);
-                  if (near(q)) que[nq++ * ng] = (uint16_t)q;
+                  const bool in = live && near(q);
+                  const uint32_t bits = (uint32_t)(__ballot(in) >> (lane & (64 - G))) & ((1u << G) - 1u);
+                  if (in) que[(nq + __popc(bits & ((1u << sub) - 1u))) * ng] = (uint16_t)q;
+                  nq += __popc(bits);
+                  if (__any(nq > brick_queue(FORM) - G)) break;
                 }
-                if (__any(nq > brick_queue(G) - 4)) break;
               }
-            } else {
-              while (w.more()) {
-                bool live;
-                const int32_t q = w.next(t, sub, live);
-                const bool in = live && near(q);
-                const uint32_t bits = (uint32_t)(__ballot(in) >> (lane & (64 - G))) & ((1u << G) - 1u);
-                if (in) que[(nq + __popc(bits & ((1u << sub) - 1u))) * ng] = (uint16_t)q;
-                nq += __popc(bits);
-                if (__any(nq > brick_queue(G) - G)) break;
+              __builtin_amdgcn_wave_barrier();   // the agent's other lanes wrote most entries
+              for (int32_t u = sub; u - sub < nq; u += G) {
+                const bool live = u < nq;
+                const int32_t q = live ? que[u * ng] : li;
+                add(q, live);
+                if (live) keep(cnt + u, q);
               }
+              cnt += nq;
+              if (!w.more()) break;
             }
-            __builtin_amdgcn_wave_barrier();   // the agent's other lanes wrote most entries
-            for (int32_t u = sub; u - sub < nq; u += G) {
-              const bool live = u < nq;
-              const int32_t q = live ? que[u * ng] : li;
-              add(q, live);
-              if (wl && live && cnt + u < a.wcap) a.wlist[(int64_t)(cnt + u) * a.ldl + row] = (int32_t)row_of(q);
-            }
-            cnt += nq;
-            if (!w.more()) break;
           }
           if (wl && sub == 0 && row - sd.row_off < N) {
             a.wlist_n[row] = cnt < a.wcap ? cnt : a.wcap;
             if (cnt > a.wcap) *a.lgate = 0;
           }
+        } else if constexpr (G == 1) {
+          brick_walk<D>(t, h, [&](int32_t q) { if (q != li) add(q, true); });
         } else {
+          BrickWalk<D, G> w(t, h, sub);
           while (w.more()) {
             bool live;
             const int32_t q = w.next(t, sub, live);
@@ -1465,10 +1508,10 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
   }
 }
 
-template <int D, class Law, int PER, int NOISE, int G, class Noise = ConstNoise>
+template <int D, class Law, int PER, int NOISE, int FORM, class Noise = ConstNoise>
 __device__ __forceinline__ void brick_body(const StageArgs& a, unsigned char* lds) {
   if (a.gate && *a.gate != a.gate_run) return;
-  brick_one<D, Law, PER, NOISE, G, false, Noise>(a, lds, xcd_tile((int)blockIdx.x, (int)gridDim.x));
+  brick_one<D, Law, PER, NOISE, FORM, false, Noise>(a, lds, xcd_tile((int)blockIdx.x, (int)gridDim.x));
 }
 
 // The sub-brick launch: the listed sub-bricks in turn.  A colony's core is a
@@ -1481,19 +1524,20 @@ __device__ __forceinline__ void sub_brick_body(const StageArgs& a, unsigned char
   if (a.gate && *a.gate != a.gate_run) return;
   const int32_t n = *a.sub_n;
   for (int32_t k = blockIdx.x; k < n; k += gridDim.x) {
-    brick_one<D, Law, PER, NOISE, 1, true, ConstNoise>(a, lds, a.sub_list[k]);
+    brick_one<D, Law, PER, NOISE, BRICK_DRAIN, true, ConstNoise>(a, lds, a.sub_list[k]);
     __syncthreads();
   }
 }
 
 // The brick kernel of a hipRTC module: nothing for a general agentODE body
-// (its row kernel walks every row).  G as for the built-in laws: a user law
-// has no reach, so every candidate takes its pair body, and in bricks cut
-// small to fill the chip one lane per agent leaves most of a block idle
-// (27,991 agents in the plane, Heun: 13.9 -> 11.9 ms for 200 steps).
-template <int D, class Law, int PER, int NOISE, class Noise, int G>
+// (its row kernel walks every row).  The form is the context's; a user law
+// has no reach, so every candidate takes its pair body and there is no queue,
+// but in bricks cut small to fill the chip one lane per agent leaves most of
+// a block idle (27,991 agents in the plane, Heun: 13.9 -> 11.9 ms for 200
+// steps with four).
+template <int D, class Law, int PER, int NOISE, class Noise, int FORM>
 __device__ __forceinline__ void user_brick(const StageArgs& a, unsigned char* lds) {
-  if constexpr (!general_body<Law>::value) brick_body<D, Law, PER, NOISE, G, Noise>(a, lds);
+  if constexpr (!general_body<Law>::value) brick_body<D, Law, PER, NOISE, FORM, Noise>(a, lds);
 }
 
 // An element at a 32-bit byte offset from a base that all lanes share (a

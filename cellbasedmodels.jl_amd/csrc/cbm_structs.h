@@ -92,8 +92,12 @@ struct alignas(8) CellRange { int32_t s, e; };
 // and the uint16 LDS index of each home row.
 constexpr int BRICK_HDR = 16;        // int32 words: total, per-wave sums; int64 at byte 48
 constexpr int BRICK_MAX_BLOCK = 256;
-// queue entries of an agent walked by g lanes
-constexpr int brick_queue(int g) { return g == 1 ? 14 : 24; }
+// How a brick's agents are walked (brick_one): one lane per agent and one walk,
+// one lane with its queue drained as it fills, or four lanes.
+constexpr int BRICK_ONE = 1, BRICK_DRAIN = 2, BRICK_FOUR = 4;
+__host__ __device__ constexpr int brick_lanes(int form) { return form == BRICK_FOUR ? 4 : 1; }
+// queue entries of an agent
+__host__ __device__ constexpr int brick_queue(int form) { return form == BRICK_ONE ? 12 : (form == BRICK_DRAIN ? 14 : 24); }
 constexpr int BRICK_WORDS = 6;       // brick table entry: sim, origin x, y, z, first bucket, end bucket
 constexpr double CL_LIST_GROW = 1.05;  // radius of the stage-2 lists, in units of the law's reach
 
@@ -101,12 +105,13 @@ __host__ __device__ constexpr int brick_halo_cells(int D, int bx, int by, int bz
   return (bx + 2) * (D > 1 ? by + 2 : 1) * (D > 2 ? bz + 2 : 1);
 }
 
-__host__ __device__ inline int64_t brick_lds_bytes(int D, bool soft, int cap, int H, int g, bool sub) {
+__host__ __device__ inline int64_t brick_lds_bytes(int D, bool soft, int cap, int H, int form, bool sub) {
   int64_t b = 4 * BRICK_HDR;
   b += (int64_t)8 * cap * (D + (soft ? 1 : 0));
   if (soft) b += (int64_t)4 * cap;
   b += (int64_t)4 * (2 * H + 1);
-  if (!sub || D > 2) b += (int64_t)2 * brick_queue(g) * (BRICK_MAX_BLOCK / g);   // sub-bricks in the plane: no filter
+  if (!sub || D > 2)   // sub-bricks in the plane: no filter
+    b += (int64_t)2 * brick_queue(form) * (BRICK_MAX_BLOCK / brick_lanes(form));
   b += (int64_t)4 * cap;      // owner and home_li, uint16 each
   return (b + 15) & ~(int64_t)15;
 }
@@ -227,7 +232,7 @@ struct StageArgs {
   int64_t brick_lds2;
   int32_t bdim2[3];
   int32_t brick_cap2;
-  int32_t brick_g;              // lanes per agent of the main brick launch (1 or 4)
+  int32_t brick_form;           // how the main brick launch walks (BRICK_ONE, BRICK_DRAIN, BRICK_FOUR)
   int32_t wcap;                 // entries per agent of wlist
   int32_t gate_run;
   int32_t fchunk;               // flattened list stage: pairs per LDS round
