@@ -479,8 +479,10 @@ static void brick_table(cbm_ctx* c, const int* bd, std::vector<int32_t>& tab) {
 // (the densest simulation's mean density; capacity when rules change the
 // population) stays within ~1.25 blocks of 256 threads, lowered while the
 // LDS for 1.2x the expected halo population would exceed 44 KiB, so that
-// three or four blocks share a CU (a denser brick is left to the
-// row-parallel stage kernel).  The density is that of
+// three or four blocks share a CU.  The smallest brick may take 64 KiB: in
+// space 44 hold 23 agents per cell and 64 hold 34, and two blocks per CU are
+// better than the row-parallel stage kernel, which has the rows of a brick
+// that is denser than its tile.  The density is that of
 // the box: an open grid's outer cells hold no agents, and counting them put
 // the tiles of small boxes under what their interior holds (120,001 soft
 // spheres, 32^3 cells: every interior brick overflowed, 123 us per stage in
@@ -547,7 +549,7 @@ static int setup_bricks(cbm_ctx* c) {
     const double want = std::min(256.0, agents / 64.0);
     while (m > mmin && cells / (double)(1 << m) < want) --m;
   }
-  const int64_t budget = 44 * 1024, budget2 = 64 * 1024;   // main bricks, sub-bricks
+  const int64_t budget = 44 * 1024, budget2 = 64 * 1024;   // main bricks; the smallest ones and sub-bricks
   // LDS bytes per staged agent and in all of a tile: the Verlet list build
   // stages positions and slots, the cell-linked stage positions (and radius
   // and fate for soft spheres); both add an owner and a home-row index
@@ -567,8 +569,10 @@ static int setup_bricks(cbm_ctx* c) {
     edges(m, bd);
     const int H = brick_halo_cells(D, bd[0], bd[1], bd[2]);
     const int64_t fixed = tile_bytes(0, H) + 16;
-    const int64_t capmax = (budget - fixed) / per;
+    int64_t capmax = (budget - fixed) / per;
     const double want = 1.2 * rho * H + 32.0;
+    if (m == mmin && want > (double)capmax)        // no smaller brick to turn to
+      capmax = (budget2 - tile_bytes(0, H, BRICK_DRAIN) - 16) / per;
     if (want <= (double)capmax || m == mmin) {
       cap = (int)std::max<int64_t>(1, std::min<int64_t>(capmax, (int64_t)std::max(256.0, want)));
       break;
