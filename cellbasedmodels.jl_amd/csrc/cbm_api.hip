@@ -1797,8 +1797,8 @@ const char* cbm_last_error(const cbm_ctx* c) { return c ? c->err.c_str() : "null
 }  // extern "C"
 
 // The hipRTC program of cbm_compile_model: the user bodies in the skeletons
-// of a model of this dimension, neighbor walk (nb, one of NB_*) and box and
-// the context's form of brick walk.
+// of a model of this dimension, neighbor walk (nb, one of NB_*) and box, with
+// the context's form of brick walk, or 0 for the program with every form.
 static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth, const char* law_body,
                                const char* noise_body, const char* rule_body, const char* medium_body, int form) {
   const int dims = m.dims;
@@ -1841,14 +1841,17 @@ static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth
                   "  cbm::user_stage<%d, %d, cbm_law_t, %d, %d, cbm_noise_t>(a);\n}\n",
                   noise, dims, nb, per, noise);
     src += inst;
-    if (nb == NB_CELL) {   // the brick-tiled cell-linked stage, run before the row kernel
-      std::snprintf(inst, sizeof(inst),
-                    "extern \"C\" __global__ __launch_bounds__(256) void cbm_user_brick_%d(cbm::StageArgs a) {\n"
-                    "  extern __shared__ unsigned char lds[];\n"
-                    "  cbm::user_brick<%d, cbm_law_t, %d, %d, cbm_noise_t, %d>(a, lds);\n}\n",
-                    noise, dims, per, noise, form);
-      src += inst;
-    }
+    if (nb == NB_CELL)     // the brick-tiled cell-linked stage, run before the row kernel
+      for (int f : {BRICK_ONE, BRICK_DRAIN, BRICK_FOUR}) {
+        if (form != f && (form != 0 || (law_body && f == BRICK_DRAIN))) continue;
+        std::snprintf(inst, sizeof(inst),
+                      "extern \"C\" __global__ __launch_bounds__(256) void cbm_user_brick_%d%s(cbm::StageArgs a) {\n"
+                      "  extern __shared__ unsigned char lds[];\n"
+                      "  cbm::user_brick<%d, cbm_law_t, %d, %d, cbm_noise_t, %d>(a, lds);\n}\n",
+                      noise, form ? "" : (f == BRICK_ONE ? "_one" : (f == BRICK_DRAIN ? "_drain" : "_four")), dims, per,
+                      noise, f);
+        src += inst;
+      }
   }
   return src;
 }
@@ -1915,7 +1918,8 @@ int cbm_compile_check(const cbm_model_desc* model, const char* law_body, const c
   const int nb = m.neighbors == CBM_FULL ? NB_FULL : (m.neighbors == CBM_CELL_LINKED ? NB_CELL : NB_LIST);
   const bool growth = m.rule == CBM_RULE_GROWTH_DIVISION || m.rule == CBM_RULE_CUSTOM;
   std::string lg;
-  const hiprtcResult r = user_compile(user_source(m, nb, growth, law_body, noise_body, rule_body, medium_body, BRICK_FOUR),
+  // every form: which one a context takes depends on its populations
+  const hiprtcResult r = user_compile(user_source(m, nb, growth, law_body, noise_body, rule_body, medium_body, 0),
                                       nullptr, &lg);
   if (log) {
     const size_t n = std::min(lg.size(), (size_t)log_cap - 1);
