@@ -75,12 +75,15 @@ __device__ __forceinline__ int64_t floor_div(double a, double b) {
 
 // --------------------------------------------- roots and quotients in range
 // The library's sqrt and division spend half of their instructions on scaling
-// and special values.  For x in [2^-200, 2^200) its square root needs neither
-// (these are its own Newton steps, so the bits are its bits), and the root's
-// last iterate is already a reciprocal good to a few ulps: one more step gives
-// r within (1/2 + 2^-34) ulp of 1/d for the price of three operations.
-// A pair's root and quotient take 18 operations so, and 3 for the range test,
-// against 29 with a quarter-rate reciprocal among them.
+// and special values.  For x in [2^-200, 2^200) the root needs neither: one
+// Goldschmidt step from the hardware's reciprocal root (2^-23 or better) and
+// two residual corrections in the manner of Markstein ("Computation of
+// elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
+// Dev. 34, 1990) round it to nearest, as the library's is rounded.  The
+// root's last iterate is already a reciprocal good to a few ulps: one more
+// step gives r within (1/2 + 2^-34) ulp of 1/d for the price of three
+// operations.  A pair's root and quotient take 18 operations so, and 5 for
+// the range test, against 29 with a quarter-rate reciprocal among them.
 struct RootInv { double d, r; };   // sqrt(x), 1/sqrt(x)
 
 __device__ __forceinline__ RootInv root_inv(double x) {
@@ -100,23 +103,32 @@ __device__ __forceinline__ RootInv root_inv(double x) {
   return o;
 }
 
-// s/d rounded to nearest, from r = 1/d as above, for s zero or 2^-800 <= |s|
-// <= 2^800.  Both residuals are exact; after the first correction q is s/d
-// within half an ulp, so the second rounds a value within (1/2 + 2^-34) 2^-53
-// ulp of s/d.  A quotient of two 53-bit numbers lies at least 2^-54 ulp from a
-// rounding boundary, and closer than that bound only for divisors whose
-// leading 34 bits are ones, with at most four numerators each.
+// s/d rounded to nearest, from r as above, for s zero or 2^-800 <= |s| <=
+// 2^800 and a d whose significand does not begin with 34 ones (root_range
+// leaves those with 20 to the library).  After the first correction q is s/d
+// within (1/2 + 2^-50) ulp; its residual is exact, so the second rounds a
+// value within (1/4 + 2^-34) 2^-53 d ulp of s/d, d scaled to [1, 2).  A
+// quotient of two 53-bit numbers lies at least 2^-53 / d ulp from the middle
+// of two doubles, which is more than that while d^2 (1 + 2^-32) < 4.
 __device__ __forceinline__ double quotient(double s, double d, double r) {
   double q = s * r;
   q = __builtin_fma(__builtin_fma(-d, q, s), r, q);
   return __builtin_fma(__builtin_fma(-d, q, s), r, q);
 }
 
-// Range tests on the high word: a squared distance in [2^-200, 2^200), a
-// length or constant (in magnitude) in [2^-100, 2^100), a constant there or 0.
+// 1/d rounded to nearest: quotient's last step, with r in q's place.
+__device__ __forceinline__ double reciprocal(double d, double r) {
+  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+
+// Range tests on the high word: a squared distance in [2^-200, 2^200) whose
+// significand does not begin with 21 ones (a root beginning with 34 of them
+// has a square beginning with 32 or more), a length or constant (in magnitude)
+// in [2^-100, 2^100), a constant there or 0.
 constexpr uint32_t ROOT_LO = (1023u - 200u) << 20, ROOT_SPAN = 400u << 20;
 __device__ __forceinline__ bool root_range(double x, uint32_t span) {
-  return (uint32_t)__double2hiint(x) - ROOT_LO < span;
+  const uint32_t h = (uint32_t)__double2hiint(x);
+  return h - ROOT_LO < span && (h & 0xFFFFFu) != 0xFFFFFu;
 }
 __device__ __forceinline__ bool plain_length(double x) {
   return ((uint32_t)__double2hiint(x) & 0x7FFFFFFFu) - ((1023u - 100u) << 20) < (200u << 20);

@@ -927,7 +927,7 @@ __global__ __launch_bounds__(256) void k_adjoint_step(AdjointArgs a) {
       } else {
         const RootInv q = root_inv(s2);   // NaN for the agent itself: never active
         d = q.d;
-        id = q.r;
+        id = reciprocal(q.d, q.r);
       }
       double phi, dphid, dth[3];
       const bool on = law(d, id, phi, dphid, dth) && in;
