@@ -128,12 +128,12 @@ __device__ __forceinline__ double reciprocal(double d, double r) {
 constexpr uint32_t ROOT_LO = (1023u - 200u) << 20, ROOT_SPAN = 400u << 20;
 __device__ __forceinline__ bool root_range(double x, uint32_t span) {
   const uint32_t h = (uint32_t)__double2hiint(x);
-  return h - ROOT_LO < span && (h & 0xFFFFFu) != 0xFFFFFu;
+  return (h - ROOT_LO < span) & ((h & 0xFFFFFu) != 0xFFFFFu);
 }
 __device__ __forceinline__ bool plain_length(double x) {
   return ((uint32_t)__double2hiint(x) & 0x7FFFFFFFu) - ((1023u - 100u) << 20) < (200u << 20);
 }
-__device__ __forceinline__ bool plain_constant(double x) { return x == 0.0 || plain_length(x); }
+__device__ __forceinline__ bool plain_constant(double x) { return (x == 0.0) | plain_length(x); }
 
 // ------------------------------------------------------------- pair laws
 // Pair magnitude s(d) of the built-in agentODE bodies with their constants
@@ -163,7 +163,8 @@ template <> struct PairLaw<LAW_LINEAR> {
   __device__ __forceinline__ double reach() const { return c; }
   // the law for d in [2^-100, 2^100): the same values (a zero's sign aside,
   // which no sum keeps); with plain() constants every s is in quotient's range
-  __device__ __forceinline__ bool plain() const { return plain_constant(k) && plain_constant(c); }
+  // (tested without branches, which would hold up the loads that follow)
+  __device__ __forceinline__ bool plain() const { return plain_constant(k) & plain_constant(c); }
   __device__ __forceinline__ bool near(double d, double& s) const {
     const double u = c - d;
     s = k * u;
@@ -191,7 +192,7 @@ template <> struct PairLaw<LAW_REP_ADH> {
   }
   __device__ __forceinline__ double reach() const { return dc; }
   __device__ __forceinline__ bool plain() const {
-    return plain_constant(k) && plain_constant(c) && plain_constant(dc) && plain_constant(a4);
+    return plain_constant(k) & plain_constant(c) & plain_constant(dc) & plain_constant(a4);
   }
   __device__ __forceinline__ bool near(double d, double& s) const {
     const double u = c - d, v = dc - d;
@@ -271,7 +272,7 @@ template <> struct PairLaw<LAW_SOFT_SPHERES> {
   }
   // the same with 1/d at hand, for plain d, r_ij and constants
   __device__ __forceinline__ bool plain() const {
-    return plain_length(mu) && plain_constant(f0[0]) && plain_constant(f0[1]) && plain_constant(f0[2]) &&
+    return plain_length(mu) & plain_constant(f0[0]) & plain_constant(f0[1]) & plain_constant(f0[2]) &
            plain_constant(f0[3]);
   }
   __device__ __forceinline__ bool near(double d, double r, double rij, int64_t fi, int64_t fj, double& s) const {

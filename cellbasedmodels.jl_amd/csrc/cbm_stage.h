@@ -372,11 +372,25 @@ __device__ __forceinline__ void gather_global(const StageArgs& a, const SimDev& 
       lp += LCH * ldl;
 #pragma unroll
       for (int u = 0; u < LCH; ++u) jn[u] = (q0 + LCH + u < cnt) ? lp[(int64_t)u * ldl] : (int32_t)i;
-      pair_terms<D, Law, PER, SOFT, LCH>(law, span, xi, px, L, hL, rad_i, rj, fate_i, fj, live, t);
+      if constexpr (has_near<Law>::value) {
+        // one pair after the other: the first one's arithmetic covers the way
+        // of the second one's position and of the indices, for which a range
+        // test of both at once would wait (device time per step: 2,305 agents
+        // in space, Euler, 17.4 -> 17.1 us; 4,001 in the plane, Heun, 23.1 ->
+        // 22.1; 12,001 in space, RK4, 36.4 -> 35.4; a million, Heun, 92.0 -> 91.4)
 #pragma unroll
-      for (int u = 0; u < LCH; ++u)
+        for (int u = 0; u < LCH; ++u) {
+          pair_term<D, Law, PER, SOFT>(law, span, xi, px[u], L, hL, live[u], t[u], rad_i, rj[u], fate_i, fj[u]);
 #pragma unroll
-        for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
+          for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
+        }
+      } else {
+        pair_terms<D, Law, PER, SOFT, LCH>(law, span, xi, px, L, hL, rad_i, rj, fate_i, fj, live, t);
+#pragma unroll
+        for (int u = 0; u < LCH; ++u)
+#pragma unroll
+          for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
+      }
     }
   } else {
     for_candidates<D, NB>(a, sd, N, i, [&](int64_t j) {
@@ -1901,11 +1915,20 @@ __device__ __forceinline__ void clv_stage_body(const StageArgs& a, unsigned char
     for (int u = 0; u < 2; ++u) jn[u] = q0 + 2 + u < n ? lp[(int64_t)(q0 + 2 + u) * ldl] : (int32_t)i;
     const bool live[2] = {q0 < n, q0 + 1 < n};
     double t[2][3];
-    pair_terms<D, Law, PER, false, 2>(law, span, xi, xj, L, hL, 0.0, nullptr, 0, nullptr, live, t);
+    if constexpr (has_near<Law>::value) {      // as in gather_global
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < 2; ++u) {
+        pair_term<D, Law, PER>(law, span, xi, xj[u], L, hL, live[u], t[u]);
 #pragma unroll
-      for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
+        for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
+      }
+    } else {
+      pair_terms<D, Law, PER, false, 2>(law, span, xi, xj, L, hL, 0.0, nullptr, 0, nullptr, live, t);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int c = 0; c < D; ++c) acc[c] = acc[c] + t[u][c];
+    }
   }
   double e2 = 0.0;
   stage_finish<D, Law, NOISE, true>(a, sd, ri.sim, i, xi, acc, upre, -1.0, &e2);
