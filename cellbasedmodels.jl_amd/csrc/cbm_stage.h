@@ -1495,11 +1495,13 @@ __device__ __forceinline__ void brick_one(const StageArgs& a, unsigned char* lds
         } else if constexpr (G == 1) {
           brick_walk<D>(t, h, [&](int32_t q) { if (q != li) add(q, true); });
         } else {
+          // a lane past the last candidate takes the agent itself: a user's law
+          // is called with distances of candidates and 0 alone
           BrickWalk<D, G> w(t, h, sub);
           while (w.more()) {
             bool live;
             const int32_t q = w.next(t, sub, live);
-            add(q, live && q != li);
+            add(live ? q : li, live && q != li);
           }
         }
       }
