@@ -1796,9 +1796,15 @@ const char* cbm_last_error(const cbm_ctx* c) { return c ? c->err.c_str() : "null
 // model's dimension, neighbor walk and boundary.
 }  // extern "C"
 
+static bool noisy_stages(const cbm_model_desc& m) {
+  return m.integrator == CBM_EM || m.integrator == CBM_EULER_HEUN;
+}
+
 // The hipRTC program of cbm_compile_model: the user bodies in the skeletons
 // of a model of this dimension, neighbor walk (nb, one of NB_*) and box, with
-// the context's form of brick walk, or 0 for the program with every form.
+// the context's form of brick walk, or 0 for the program with every form.  A
+// context's integrator runs either the noisy stages or the others, and its
+// program holds those alone: half of the compile.
 static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth, const char* law_body,
                                const char* noise_body, const char* rule_body, const char* medium_body, int form) {
   const int dims = m.dims;
@@ -1832,10 +1838,12 @@ static std::string user_source(const cbm_model_desc& m, int nb_kind, bool growth
   src += noise_body ? "using cbm_noise_t = cbm::UserNoise;\n" : "using cbm_noise_t = cbm::ConstNoise;\n";
   // the same skeletons as the built-in laws: no neighbor walk without a law
   const bool walk = m.law != CBM_LAW_NONE;
+  const int only = form == 0 ? -1 : (noisy_stages(m) ? 1 : 0);
   const int nb = walk ? nb_kind : NB_FULL;
   const int per = walk && m.periodic ? 1 : 0;
   char inst[512];
   for (int noise = 0; stages && noise < 2; ++noise) {
+    if (only >= 0 && noise != only) continue;
     std::snprintf(inst, sizeof(inst),
                   "extern \"C\" __global__ __launch_bounds__(256) void cbm_user_stage_%d(cbm::StageArgs a) {\n"
                   "  cbm::user_stage<%d, %d, cbm_law_t, %d, %d, cbm_noise_t>(a);\n}\n",
@@ -1987,7 +1995,7 @@ int cbm_compile_model(cbm_ctx* c, const char* law_body, const char* noise_body, 
     return fail(c, CBM_ERR_CONFIG, "a law body is required with law CBM_LAW_CUSTOM and only then");
   if ((c->m.rule == CBM_RULE_CUSTOM) != (rule_body != nullptr))
     return fail(c, CBM_ERR_CONFIG, "a rule body is required with rule CBM_RULE_CUSTOM and only then");
-  if (noise_body && c->m.integrator != CBM_EM && c->m.integrator != CBM_EULER_HEUN)
+  if (noise_body && !noisy_stages(c->m))
     return fail(c, CBM_ERR_CONFIG, "an agentSDE body needs the EM or EulerHeun integrator");
   if (medium_body && !c->medium) return fail(c, CBM_ERR_CONFIG, "a mediumODE body needs a medium (medium_n)");
   if (!law_body && !noise_body && !rule_body && !medium_body) return fail(c, CBM_ERR_ARG, "nothing to compile");
@@ -2037,12 +2045,10 @@ int cbm_compile_model(cbm_ctx* c, const char* law_body, const char* noise_body, 
     }
   }
   if (stages) {
-    HIPCHK(c, hipModuleGetFunction(&c->user_fn[0], c->user_mod, "cbm_user_stage_0"));
-    HIPCHK(c, hipModuleGetFunction(&c->user_fn[1], c->user_mod, "cbm_user_stage_1"));
-  }
-  if (stages && nb == NB_CELL) {
-    HIPCHK(c, hipModuleGetFunction(&c->user_brick[0], c->user_mod, "cbm_user_brick_0"));
-    HIPCHK(c, hipModuleGetFunction(&c->user_brick[1], c->user_mod, "cbm_user_brick_1"));
+    const int k = noisy_stages(c->m) ? 1 : 0;
+    const std::string q = std::to_string(k);
+    HIPCHK(c, hipModuleGetFunction(&c->user_fn[k], c->user_mod, ("cbm_user_stage_" + q).c_str()));
+    if (nb == NB_CELL) HIPCHK(c, hipModuleGetFunction(&c->user_brick[k], c->user_mod, ("cbm_user_brick_" + q).c_str()));
   }
   c->user_nb = nb;
   c->user_noise = noise_body != nullptr;
@@ -2199,7 +2205,8 @@ int cbm_neighbors(cbm_ctx* c) {
 
 int cbm_step(cbm_ctx* c, int64_t nsteps) {
   if (!c || nsteps < 0) return CBM_ERR_ARG;
-  if (c->m.law == CBM_LAW_CUSTOM && !c->user_fn[0]) return fail(c, CBM_ERR_CONFIG, "law CBM_LAW_CUSTOM: call cbm_compile first");
+  if (c->m.law == CBM_LAW_CUSTOM && !c->user_fn[noisy_stages(c->m) ? 1 : 0])
+    return fail(c, CBM_ERR_CONFIG, "law CBM_LAW_CUSTOM: call cbm_compile first");
   if (c->m.rule == CBM_RULE_CUSTOM && !c->user_rule[0])
     return fail(c, CBM_ERR_CONFIG, "rule CBM_RULE_CUSTOM: call cbm_compile_model with a rule body first");
   c->last_launches = 0;
@@ -2966,7 +2973,7 @@ int cbm_autotune(cbm_ctx* c, const char* cache_path, int32_t* block) {
     a.U[v] = statecol(c, v, false);
     a.out[v] = c->h[0][v] ? c->h[0][v] : statecol(c, v, true);
   }
-  a.kind = ST_HEUN1;
+  a.kind = c->m.law == CBM_LAW_CUSTOM && noisy_stages(c->m) ? ST_EM : ST_HEUN1;   // a compiled law has its integrator's kind
   const int cand[3] = {64, 128, 256};
   float best_ms = 1e30f;
   int best = c->block;
