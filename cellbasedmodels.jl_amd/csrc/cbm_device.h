@@ -105,7 +105,7 @@ __device__ __forceinline__ RootInv root_inv(double x) {
 
 // s/d rounded to nearest, from r as above, for s zero or 2^-800 <= |s| <=
 // 2^800 and a d whose significand does not begin with 34 ones (root_range
-// leaves those with 20 to the library).  After the first correction q is s/d
+// leaves those with 21 to the library).  After the first correction q is s/d
 // within (1/2 + 2^-50) ulp; its residual is exact, so the second rounds a
 // value within (1/4 + 2^-34) 2^-53 d ulp of s/d, d scaled to [1, 2).  A
 // quotient of two 53-bit numbers lies at least 2^-53 / d ulp from the middle

@@ -88,7 +88,7 @@ struct alignas(8) CellRange { int32_t s, e; };
 // LDS of one brick block: a header of int32 words, then D position arrays
 // (and radius for soft spheres) of cap doubles, int32 fate (soft spheres),
 // the halo cells' LDS offsets (H + 1) and first rows (H), the queues of kept
-// candidates (one per four lanes), the uint16 halo cell of each staged agent
+// candidates (one per agent under way), the uint16 halo cell of each staged agent
 // and the uint16 LDS index of each home row.
 constexpr int BRICK_HDR = 16;        // int32 words: total, per-wave sums; int64 at byte 48
 constexpr int BRICK_MAX_BLOCK = 256;
