@@ -746,7 +746,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a) {
 // Setting up and finishing a rod by one lane of G costs what the shorter
 // series saves where wavefronts abound, so there is no other form.  20,011
 // rods of 45 candidates each: 161 us per stage with a lane per rod, 37 us now;
-// steps of 200,003 and 1,000,003 rods 0.90 and 2.8 ms, now 0.66 and 2.7.
+// steps of 200,003 (Heun) and 1,000,003 (Euler) rods 0.90 and 2.8 ms, now 0.66
+// and 2.7.
 template <int NB> struct rod_lanes { static constexpr int value = NB == NB_LIST ? 8 : 16; };   // lists are shorter
 
 template <int NB>
